@@ -334,7 +334,7 @@ __global__ __launch_bounds__(kTThreads) void k_attn_t(AttnParams p) {
     for (int t = 0; t < QT; t++) {
         const int q = ((qb * kTWaves + wave) * QT + t) * 16 + r16;
         const float l = xsum4(S.l[t]);  // the query's 4 partial sums
-        if (q < nq) attn_emit<HD>(p, s, h * p.n_rep + q % p.n_rep, q / p.n_rep, g, S.o[t], S.m[t], l);
+        if (q < nq) attn_emit<HD, false, 1>(p, s, h * p.n_rep + q % p.n_rep, q / p.n_rep, g, S.o[t], S.m[t], l);
     }
 }
 
@@ -400,7 +400,7 @@ template <int NS> __global__ __launch_bounds__(kCombThreads) void k_attn_combine
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         const int64_t e = (int64_t)head * HD + 8 * c + 4 * k;
-        *(uintx2 *)(p.out16 + (int64_t)m * p.out_ld + frag_index(e)) =
+        *(uintx2 *)(p.out16 + act_index(m, e, p.out_ld, p.M > 16)) =
             uintx2{(uint32_t)f2h(acc[4 * k] / W) | ((uint32_t)f2h(acc[4 * k + 2] / W) << 16),
                    (uint32_t)f2h(acc[4 * k + 1] / W) | ((uint32_t)f2h(acc[4 * k + 3] / W) << 16)};
     }

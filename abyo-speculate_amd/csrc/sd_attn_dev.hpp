@@ -285,18 +285,17 @@ __device__ __forceinline__ void attn_step(AttnState<HD, QT> &S, KvStep<HD> &b, K
 // order); otherwise o / l as fp16 and (m, l) for the merge of the splits,
 // which weighs split s by l_s * exp2(m_s - max m).  DEV: the partials are
 // stored at device scope, for a merge inside the same launch.
-template <int HD, bool DEV = false>
+template <int HD, bool DEV = false, int TILED = 0>
 __device__ __forceinline__ void attn_emit(const AttnParams &p, int s, int head, int m, int g,
                                           const floatx4 (&o)[HD / 16], float mq, float l) {
     const float inv = 1.0f / l;
     if (p.nsplit == 1) {
+        // dims 4g .. 4g + 3 sit in fragment slots f, f + 2, f + 1, f + 3
 #pragma unroll
         for (int dt = 0; dt < HD / 16; dt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t k = (int64_t)head * HD + dt * 16 + 4 * g + i;
-                p.out16[(int64_t)m * p.out_ld + frag_index(k)] = f2h(o[dt][i] * inv);
-            }
+            *(uintx2 *)(p.out16 + act_index(m, (int64_t)head * HD + dt * 16 + 4 * g, p.out_ld, TILED)) =
+                uintx2{(uint32_t)f2h(o[dt][0] * inv) | ((uint32_t)f2h(o[dt][2] * inv) << 16),
+                       (uint32_t)f2h(o[dt][1] * inv) | ((uint32_t)f2h(o[dt][3] * inv) << 16)};
         return;
     }
     const int64_t pi = ((int64_t)s * p.n_heads + head) * p.M + m;

@@ -58,6 +58,21 @@ __host__ __device__ inline int frag_slot(int e) {
 }
 __host__ __device__ inline int64_t frag_index(int64_t k) { return (k & ~int64_t(255)) + frag_slot((int)(k & 255)); }
 
+// Above 16 rows activations are kept in MFMA operand order instead: per tile of
+// 32 tokens and superblock 16 operands of v_mfma_f32_32x32x16_f16, operand 2 c +
+// (g >> 1) holding for lane (token & 31) + 32 * (g & 1) the 8 slots of (c, g).
+// fi: the element's fragment-order index in its row (frag_index); ld: row length.
+__host__ __device__ inline int64_t xt_index(int64_t m, int64_t fi, int ld) {
+    const int f = (int)(fi & 255);
+    return (((m >> 5) * (ld >> 8) + (fi >> 8)) * 16 + (f >> 5) * 2 + ((f >> 4) & 1)) * 512 +
+           ((m & 31) + 32 * ((f >> 3) & 1)) * 8 + (f & 7);
+}
+// where element k of row m of a matmul's input lives: operand order (above 16
+// rows) or the row's own fragment order
+__host__ __device__ inline int64_t act_index(int64_t m, int64_t k, int ld, int tiled) {
+    return tiled ? xt_index(m, frag_index(k), ld) : m * ld + frag_index(k);
+}
+
 // ---- KV cache layout ----------------------------------------------------
 // The cache holds, per (layer, K/V, kv head) "stream", cap positions x hd
 // fp16 values (cap a multiple of 32), blocked so that every MFMA operand the

@@ -22,7 +22,7 @@ namespace sd {
 template <int NV, int NT>  // NT threads, NV float4 vectors per thread: K = 4 * NT * NV
 __global__ __launch_bounds__(NT) void k_rmsnorm(float *x, const float *w, int K, float eps, uint16_t *out16,
                                                 int ld16, float *out32, const float *part, int nks,
-                                                int64_t pstride) {
+                                                int64_t pstride, int tiled) {
     const int m = blockIdx.x, t = threadIdx.x;
     float4 *row = (float4 *)(x + (int64_t)m * K);
     const float4 *wv = (const float4 *)w;
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(NT) void k_rmsnorm(float *x, const float *w, int K,
             // elements k .. k+3 sit in fragment slots f, f+2, f+1, f+3: one 8-byte store
             const uint32_t lo = (uint32_t)f2h(y[0]) | ((uint32_t)f2h(y[2]) << 16);
             const uint32_t hi = (uint32_t)f2h(y[1]) | ((uint32_t)f2h(y[3]) << 16);
-            *(uint2 *)(out16 + (int64_t)m * ld16 + frag_index(k)) = make_uint2(lo, hi);
+            *(uint2 *)(out16 + act_index(m, k, ld16, tiled)) = make_uint2(lo, hi);
         }
         if (out32) *(float4 *)(out32 + (int64_t)m * K + k) = make_float4(y[0], y[1], y[2], y[3]);
     }
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(NT) void k_rmsnorm(float *x, const float *w, int K,
 // generic K (multiple of 4): strided loop
 __global__ __launch_bounds__(256) void k_rmsnorm_any(float *x, const float *w, int K, float eps, uint16_t *out16,
                                                      int ld16, float *out32, const float *part, int nks,
-                                                     int64_t pstride) {
+                                                     int64_t pstride, int tiled) {
     const int m = blockIdx.x;
     float *row = x + (int64_t)m * K;
     if (nks > 1) {
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_any(float *x, const float *w, i
     const float mrms = sqrtf(red[0] / (float)K + eps);
     for (int k = threadIdx.x; k < K; k += 256) {
         const float y = row[k] / mrms * w[k];
-        if (out16) out16[(int64_t)m * ld16 + frag_index(k)] = f2h(y);
+        if (out16) out16[act_index(m, k, ld16, tiled)] = f2h(y);
         if (out32) out32[(int64_t)m * K + k] = y;
     }
 }
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(NT) void k_resid_u(float *x, const float *w, int K,
     // elements k .. k+3 sit in fragment slots f, f+2, f+1, f+3: one 8-byte store
     const uint32_t lo = (uint32_t)f2h(v.x * wv.x) | ((uint32_t)f2h(v.z * wv.z) << 16);
     const uint32_t hi = (uint32_t)f2h(v.y * wv.y) | ((uint32_t)f2h(v.w * wv.w) << 16);
-    *(uint2 *)(out16 + (int64_t)m * ld16 + frag_index(k)) = make_uint2(lo, hi);
+    *(uint2 *)(out16 + act_index(m, k, ld16, 1)) = make_uint2(lo, hi);
     float ss = v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
     ss += __shfl_xor(ss, 1);
     ss += __shfl_xor(ss, 2);
@@ -200,11 +200,11 @@ __global__ __launch_bounds__(256) void k_norm_u(const float *x, const float *w, 
 }
 
 // f32 rows -> fp16 fragment layout (hidden states handed to apply_lm_head)
-__global__ void k_to_frag16(const float *x, int K, uint16_t *out16, int ld16) {
+__global__ void k_to_frag16(const float *x, int K, uint16_t *out16, int ld16, int tiled) {
     const int m = blockIdx.y;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= K) return;
-    out16[(int64_t)m * ld16 + frag_index(k)] = f2h(x[(int64_t)m * K + k]);
+    out16[act_index(m, k, ld16, tiled)] = f2h(x[(int64_t)m * K + k]);
 }
 
 // ---- argmax over per-workgroup partials (first max wins, NaN/-inf skipped) ----
@@ -304,9 +304,8 @@ __global__ __launch_bounds__(256) void k_keep_kv_tail(uint16_t *kv, int64_t stre
 
 // ---- launchers ----
 void launch_rmsnorm(float *x, const float *w, int M, int K, float eps, uint16_t *out16, int ld16, float *out32,
-                    hipStream_t st, const float *part, int nks) {
-    const int64_t ps = (int64_t)M * K;
-#define SD_RMS(KERN, NT) hipLaunchKernelGGL(KERN, dim3(M), dim3(NT), 0, st, x, w, K, eps, out16, ld16, out32, part, nks, ps)
+                    hipStream_t st, const float *part, int nks, int64_t ps, int tiled) {
+#define SD_RMS(KERN, NT) hipLaunchKernelGGL(KERN, dim3(M), dim3(NT), 0, st, x, w, K, eps, out16, ld16, out32, part, nks, ps, tiled)
     // one float4 per thread (and slice) where K allows: the row's loads spread
     // over 16 waves
     switch (K) {
@@ -337,7 +336,7 @@ void launch_resid_u(float *x, const float *w, int M, int K, const float *part, i
     else hipLaunchKernelGGL(k_resid_u<64>, dim3(M, nb), dim3(64), 0, st, x, w, K, part, nks, ps, out16, ld16, ssq);
 }
 void launch_to_frag16(const float *x, int M, int K, uint16_t *out16, int ld16, hipStream_t st) {
-    hipLaunchKernelGGL(k_to_frag16, dim3((K + 255) / 256, M), dim3(256), 0, st, x, K, out16, ld16);
+    hipLaunchKernelGGL(k_to_frag16, dim3((K + 255) / 256, M), dim3(256), 0, st, x, K, out16, ld16, M > 16 ? 1 : 0);
 }
 void launch_argmax_reduce(const float *pv, const int *pi, int nwg, int M, int *out, hipStream_t st) {
     hipLaunchKernelGGL(k_argmax_reduce, dim3(M), dim3(256), 0, st, pv, pi, nwg, out);

@@ -15,7 +15,10 @@ struct BackendError : std::runtime_error {
 // Device address of this GPU's file-scope scratch array (kNoAllocScratchBytes),
 // resolved with hipGetSymbolAddress on the first call for `device`, which must
 // be the current device; later calls return the kept address.
-constexpr size_t kNoAllocScratchBytes = (size_t)4 << 20;
+// Calls stage at most kNoAllocMaxBytes of rows; above 16 rows they fill whole
+// tiles of 32 rows, less than twice as many.
+constexpr size_t kNoAllocMaxBytes = (size_t)4 << 20;
+constexpr size_t kNoAllocScratchBytes = 2 * kNoAllocMaxBytes;
 void *noalloc_scratch(int device);
 
 // ---- sd_synth.hip ----
@@ -63,11 +66,11 @@ struct GemmParams {
     GemmSeg seg[4];
     int nseg;
     int ntiles;              // total 16-row tiles (sum over segments)
-    const uint16_t *xp;      // fp16 activations, fragment layout, [Mpad][K]
+    const uint16_t *xp;      // fp16 activations: fragment order [M][K], above 16 rows operand order (xt_index)
     int K;
     int M;
     int mode;
-    uint16_t *act;           // GM_SWIGLU: fp16 fragment-layout output [Mpad][act_ld]
+    uint16_t *act;           // GM_SWIGLU: fp16 output, the layout of the next matmul's xp
     int act_ld;
     float *amax_v;           // GM_LOGITS: per (token, workgroup) argmax partials
     int *amax_i;
@@ -109,5 +112,10 @@ struct LaunchTiming {
 int launch_qgemm(const GemmParams &p, hipStream_t st, const LaunchTiming &tm = LaunchTiming{});
 int qgemm_workgroups(const GemmParams &p);
 int qgemm_slices(const GemmParams &p);  // 1 when the output is written directly
+
+// ---- sd_qwide.hip: the same above 16 rows (launch_qgemm dispatches) ----
+void launch_qwide(const GemmParams &p, hipStream_t st, const LaunchTiming &tm);
+int qwide_slices(const GemmParams &p);
+int qwide_slots(const GemmParams &p);  // argmax partials per token of a GM_LOGITS launch
 
 }  // namespace sd

@@ -135,7 +135,7 @@ void Model::alloc_buffers() {
     logits = dalloc<float>((size_t)Mx * c.vocab);
     hidden_out = dalloc<float>((size_t)Mx * c.hidden);
     last_row = dalloc<float>((size_t)c.vocab);
-    amax_ld = c.vocab / 16;
+    amax_ld = (c.vocab + 127) / 128 * 8;
     amax_v = dalloc<float>((size_t)Mx * amax_ld);
     amax_i = dalloc<int>((size_t)Mx * amax_ld);
     argmax = dalloc<int>(Mx);
@@ -473,9 +473,11 @@ void Model::qmatmul_into(int layer, int kind, const float *x_dev, int M, float *
     DevTensor &t = slot(*this, layer, kind);
     if (!t.set() || t.fmt == F32) throw ArgError("qmatmul needs a quantised matrix tensor");
     if (M < 1 || M > 128) throw ArgError("rows must be in [1, 128]");
-    if ((size_t)M * t.K * 2 > staging_bytes)
+    if ((size_t)M * t.K * 2 > kNoAllocMaxBytes)
         throw ArgError("rows * K * 2 = " + std::to_string((size_t)M * t.K * 2) + " bytes of staged activations exceed the " +
-                       std::to_string(staging_bytes) + "-byte scratch");
+                       std::to_string(kNoAllocMaxBytes) + "-byte scratch");
+    if ((size_t)(M > 16 ? (M + 31) / 32 * 32 : M) * t.K * 2 > staging_bytes)  // whole 32-row tiles
+        throw BackendError("staging too small");
     hipStream_t s = stream ? stream : st;
     launch_to_frag16(x_dev, M, t.K, (uint16_t *)staging, t.K, s);
     GemmParams p{};  // allow_split = 0: no split-K partials
@@ -612,6 +614,8 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
     // matmuls); not while per-layer hidden states are collected
     const int split_ok = collect.empty() ? 1 : 0;
     int pend = 1;  // K slices of the last residual matmul not yet added to h
+    const int64_t ps = (int64_t)M * H;  // their stride
+    const int tiled = M > 16;           // the layout of the matmuls' inputs (act_index)
     // Up to 16 rows the RMSNorms and RoPE live in the matmul epilogues: the
     // residual matmuls (wo, ffn_down) also write u = fp16(h * w_next_norm)
     // and per-tile sums of h^2, the next matmul scales its outputs by
@@ -638,7 +642,7 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
         if (spread)
             launch_resid_u(h, (const float *)L[K_ATTN_NORM].d, M, H, qg_part, pend, xp, xp_ld, ssq, st);
         else if (!fused)
-            launch_rmsnorm(h, (const float *)L[K_ATTN_NORM].d, M, H, c.rms_eps, xp, xp_ld, nullptr, st, qg_part, pend);
+            launch_rmsnorm(h, (const float *)L[K_ATTN_NORM].d, M, H, c.rms_eps, xp, xp_ld, nullptr, st, qg_part, pend, ps, tiled);
         int nks_qkv;
         bool qa_launched = false;
         AttnParams a{};
@@ -788,7 +792,7 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
         if (spread)
             launch_resid_u(h, (const float *)L[K_FFN_NORM].d, M, H, qg_part, pend, xp, xp_ld, ssq, st);
         else if (!fused)
-            launch_rmsnorm(h, (const float *)L[K_FFN_NORM].d, M, H, c.rms_eps, xp, xp_ld, nullptr, st, qg_part, pend);
+            launch_rmsnorm(h, (const float *)L[K_FFN_NORM].d, M, H, c.rms_eps, xp, xp_ld, nullptr, st, qg_part, pend, ps, tiled);
         {
             GemmParams p{};
             gemm_workspace(p);
@@ -835,17 +839,20 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
                 SD_HIP_CHECK(hipMemcpyAsync(collect_buf + ci * H, h + (size_t)(M - 1) * H, H * 4,
                                             hipMemcpyDeviceToDevice, st));
     }
-    // the lm_head over all rows reads u and scales; other requests normalise here
+    // The lm_head over all rows reads u and scales, or the normalised rows;
+    // other requests normalise the last row only (hidden_out row 0), which
+    // above 16 rows becomes row 0 of xp in the one-row layout
+    const float *wn = (const float *)gw[K_OUTPUT_NORM].d;
     const bool spread_head = spread && logits_mode == 2;
-    if (spread_head) {
-        launch_resid_u(h, (const float *)gw[K_OUTPUT_NORM].d, M, H, qg_part, pend, xp, xp_ld, ssq, st);
-        if (want_hidden)  // h is complete: the final-norm hidden rows only
-            launch_rmsnorm(h, (const float *)gw[K_OUTPUT_NORM].d, M, H, c.rms_eps, nullptr, 0, hidden_out, st);
-    } else if (!fused) {
-        launch_rmsnorm(h, (const float *)gw[K_OUTPUT_NORM].d, M, H, c.rms_eps, xp, xp_ld,
-                       want_hidden ? hidden_out : nullptr, st, qg_part, pend);
-    } else if (want_hidden) {  // the final-norm hidden rows only; the lm_head input is already in xp
-        launch_rmsnorm(h, (const float *)gw[K_OUTPUT_NORM].d, M, H, c.rms_eps, nullptr, 0, hidden_out, st);
+    if (logits_mode == 2) {
+        if (spread_head) launch_resid_u(h, wn, M, H, qg_part, pend, xp, xp_ld, ssq, st);
+        if (want_hidden || !(spread || fused))
+            launch_rmsnorm(h, wn, M, H, c.rms_eps, spread || fused ? nullptr : xp, xp_ld,
+                           want_hidden ? hidden_out : nullptr, st, qg_part, spread ? 1 : pend, ps, tiled);
+    } else if (want_hidden || (!fused && logits_mode == 1)) {
+        const int64_t r0 = (int64_t)(M - 1) * H;
+        launch_rmsnorm(h + r0, wn, 1, H, c.rms_eps, fused ? nullptr : xp, xp_ld, want_hidden ? hidden_out : nullptr, st,
+                       qg_part + r0, pend, ps, 0);
     }
     logits_rows_last = 0;
     if (logits_mode != 0) {
@@ -856,7 +863,7 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
         p.seg[0] = seg_of(W, 0, logits, c.vocab, 0, nullptr);
         p.nseg = 1;
         p.ntiles = W.rows / 16;
-        p.xp = xp + (logits_mode == 1 ? (size_t)(M - 1) * xp_ld : 0);
+        p.xp = xp + (logits_mode == 1 && fused ? (size_t)(M - 1) * xp_ld : 0);
         p.K = H;
         p.M = rows;
         p.mode = GM_LOGITS;
@@ -1243,7 +1250,6 @@ void Decoder::observe_returning_last_hidden(const uint32_t *ids, size_t n, float
     std::vector<int> tk, pos;
     std::vector<uint64_t> mw;
     int nw;
-    int lastM = 1;
     while (done < n) {
         const int M = (int)std::min<size_t>(m.cfg.max_batch, n - done);
         tk.assign(ids + done, ids + done + M);
@@ -1253,11 +1259,10 @@ void Decoder::observe_returning_last_hidden(const uint32_t *ids, size_t n, float
         m.forward(tk.data(), pos.data(), mw.data(), nw, M, cache_len, 0, done + M == n, {}, nullptr);
         cache_len += M;
         done += M;
-        lastM = M;
     }
     history.insert(history.end(), ids, ids + n);
     if (out)
-        SD_HIP_CHECK(hipMemcpyAsync(out, m.hidden_out + (size_t)(lastM - 1) * m.cfg.hidden, (size_t)m.cfg.hidden * 4,
+        SD_HIP_CHECK(hipMemcpyAsync(out, m.hidden_out, (size_t)m.cfg.hidden * 4,
                                     hipMemcpyDeviceToHost, m.st));
     m.sync();
 }

@@ -4,19 +4,17 @@
 // (crates/speculate/src/model/quantized_llama_local.rs:47-49 MLP, :73-90 Q/K/V,
 // :135 wo, :317 lm_head; quantized_qwen2_local.rs:41-44, 71-82, 138, 315).
 //
-// Both kernels multiply 16 weight rows x 32 K by 32 K x 16 tokens (fp16
-// activations in fragment order) with v_mfma_f32_16x16x32_f16 and accumulate
-// in f32.
+// Up to 16 rows (decode, linear verify); launch_qgemm hands larger inputs to
+// the kernel of sd_qwide.hip.  16 weight rows x 32 K by 32 K x 16 tokens (fp16
+// activations in fragment order) go through v_mfma_f32_16x16x32_f16 and
+// accumulate in f32.
 //
-//  * k_qmm (M <= 16, the linear-verify shape): one 16-token tile, products
-//    transposed (tokens x rows).  A workgroup owns RT row tiles and KW waves
-//    that split the K superblocks (wave w takes w, w+KW, ...), each with the
-//    next superblock's weights and activations in flight; KW is chosen per
-//    matrix so that every launch puts thousands of waves on the 256 CUs.
-//    Q4_K / Q5_K weights enter the MFMA as exact integers (see kquant_int).
-//  * k_qgx (M > 16, tree and prefill shapes): 4 waves share each superblock's
-//    activations through LDS; CT token tiles per wave reuse every dequantised
-//    weight fragment CT times.
+//  * k_qmm: one 16-token tile, products transposed (tokens x rows).  A
+//    workgroup owns RT row tiles and KW waves that split the K superblocks
+//    (wave w takes w, w+KW, ...), each with the next superblock's weights and
+//    activations in flight; KW is chosen per matrix so that every launch puts
+//    thousands of waves on the 256 CUs.  Q4_K / Q5_K weights enter the MFMA as
+//    exact integers (see kquant_int).
 //
 // Accumulation order is fixed by the matrix alone: per wave, superblocks in
 // increasing order and chunks c = 0..7 in order; across waves, partial sums
@@ -24,13 +22,11 @@
 // (rows, K), never on M, so row i of an M-row call (M <= 16) equals the M=1
 // call bit for bit.
 //
-// Dequantisation to fp16 (k_qgx, and Q6_K / Q8_0 in k_qmm): a code is OR'ed
-// into the mantissa of 1024.0h (0x6400 | q == 1024 + q) or, for a code already
-// at bits 4-7, of 64.0h (0x5400 | q << 4 == 64 + q).  Q6_K: q - 32 exactly,
-// times the fp16 sub-block scale fp16(d * sc) in one v_pk_mul_f16.  Q8_0: q
-// exactly, times the fp16 block scale in one v_pk_mul_f16.  Q4_K / Q5_K (k_qgx): q exactly, then one
-// v_pk_fma_f16 with the sub-block's fp16 scale and min, round_f16(q * s16 -
-// m16) where s16 = fp16(d * sc) and m16 = fp16(dmin * m).
+// Dequantisation to fp16 (Q6_K / Q8_0): a code is OR'ed into the mantissa of
+// 1024.0h (0x6400 | q == 1024 + q) or, for a code already at bits 4-7, of
+// 64.0h (0x5400 | q << 4 == 64 + q).  Q6_K: q - 32 exactly, times the fp16
+// sub-block scale fp16(d * sc) in one v_pk_mul_f16.  Q8_0: q exactly, times
+// the fp16 block scale in one v_pk_mul_f16.
 #include <hip/hip_ext.h>
 
 #include "sd_attn_dev.hpp"
@@ -144,27 +140,6 @@ __device__ __forceinline__ KInt kquant_int(const uintx4 &hdr, int g) {
     return k;
 }
 
-// fp16 pairs of one lane's two sub-blocks (see QFmt<Q4_K>::S)
-struct KS16 {
-    uint32_t s0, m0, s1, m1;
-};
-__device__ __forceinline__ KS16 kquant_s16(const uintx4 &hdr, int g) {
-    const float d = h2f((uint16_t)(hdr.x & 0xffffu)), dmin = h2f((uint16_t)(hdr.x >> 16));
-    int sc[2], mn[2];
-    kquant_ints(hdr, g, sc, mn);
-    KS16 k;
-    k.s0 = h2pair(d * (float)sc[0]);  // exact f32 products, one rounding each
-    k.m0 = h2pair(-(dmin * (float)mn[0]));
-    k.s1 = h2pair(d * (float)sc[1]);
-    k.m1 = h2pair(-(dmin * (float)mn[1]));
-    return k;
-}
-// codes (off + q) -> round_f16(q * s + nm), q exact
-__device__ __forceinline__ uint32_t qsm(uint32_t p, uint32_t off, uint32_t s, uint32_t nm) {
-    const half2v q = __builtin_bit_cast(half2v, p) + __builtin_bit_cast(half2v, off);
-    return pkfma(__builtin_bit_cast(uint32_t, q), s, nm);
-}
-
 template <> struct QFmt<Q4_K> {
     typedef LaneQ4K D;
     static constexpr bool kInt = true;
@@ -175,12 +150,6 @@ template <> struct QFmt<Q4_K> {
         return as_half8(pkfma(p[0], s.s0, s.c0), pkfma(p[1], s.s0, s.c0), pkfma(p[2], s.s1, s.c1),
                         pkfma(p[3], s.s1, s.c1));
     }
-    // Above 16 rows (weights as the MFMA's fp16 operand): the sub-block
-    // scales as fp16 pairs, s = fp16(d * sc) and -m = -fp16(dmin * mn); a code
-    // (1024 + q or 64 + q) minus its offset is q exactly, and one
-    // v_pk_fma_f16 gives round_f16(q * s - m) (a single rounding of the exact
-    // q * s - m).  Two packed instructions per pair of weights.
-    typedef KS16 S;
     static __device__ __forceinline__ void load(D &r, const WRow &w, int nsb, int sb, int g) {
         const int lane = threadIdx.x & 63;
         const uint32_t so = tb_off(w, sb, D::TBB);
@@ -188,18 +157,10 @@ template <> struct QFmt<Q4_K> {
         r.q0 = bld16(w.rs, D::off_q0(lane), so);
         r.q1 = bld16(w.rs, D::off_q1(lane), so);
     }
-    static __device__ __forceinline__ S scales(const D &r, int g) { return kquant_s16(r.hdr, g); }
-    static __device__ __forceinline__ half8 frag(const D &r, const S &s, int g, int c) {
-        uint32_t p[4];
-        r.codes(g, c, p);
-        return as_half8(qsm(p[0], kOff1024, s.s0, s.m0), qsm(p[1], kOff1024, s.s0, s.m0),
-                        qsm(p[2], kOff64, s.s1, s.m1), qsm(p[3], kOff64, s.s1, s.m1));
-    }
 };
 
 template <> struct QFmt<Q5_K> {
     typedef LaneQ5K D;
-    typedef QFmt<Q4_K>::S S;
     static constexpr bool kInt = true;
     static __device__ __forceinline__ KInt iscales(const D &r, int g) { return kquant_int(r.hdr, g); }
     static __device__ __forceinline__ half8 ifrag(const D &r, const KInt &s, int g, int c) {
@@ -215,13 +176,6 @@ template <> struct QFmt<Q5_K> {
         r.qh = bld8(w.rs, D::off_qh(lane), so);
         r.q0 = bld16(w.rs, D::off_q0(lane), so);
         r.q1 = bld16(w.rs, D::off_q1(lane), so);
-    }
-    static __device__ __forceinline__ S scales(const D &r, int g) { return kquant_s16(r.hdr, g); }
-    static __device__ __forceinline__ half8 frag(const D &r, const S &s, int g, int c) {
-        uint32_t p[4];
-        r.codes(g, c, p);
-        return as_half8(qsm(p[0], kOff1024, s.s0, s.m0), qsm(p[1], kOff1024, s.s0, s.m0),
-                        qsm(p[2], kOff64, s.s1, s.m1), qsm(p[3], kOff64, s.s1, s.m1));
     }
 };
 
@@ -917,226 +871,6 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2)
     attn_wg<HD, true>(a, h, r % a.nsplit, r / a.nsplit, w);
 }
 
-// ==========================================================================
-// M > 16 (tree and prefill shapes).  A workgroup of 4 waves owns a row block
-// -- 4 x RW row tiles, or for gate/up 4 features' gate and up tiles -- and one
-// K slice.  The slice's activations are staged superblock by superblock in
-// LDS, so each activation byte is fetched from L2 once per workgroup and read
-// by all 4 waves (reading them per wave from L1 made the M = 60 launches L2
-// bound); the weights stream into registers one superblock ahead.  With more
-// than one K slice the launch writes per-slice partial sums and the kernel
-// that consumes the output adds them (GM_STORE / GM_RESID callers only).
-// ==========================================================================
-constexpr int XG_WAVES = 4;
-constexpr int XG_PITCH = 528;  // bytes per staged token row: 512 + 16 keeps ds_read_b128 conflict free
-
-template <int CT> struct XStage {
-    uintx4 v[2 * CT];  // CT*16 rows x 32 16-byte pieces over 256 threads
-};
-
-// the activations of superblock sb (a negative sb loads nothing)
-template <int CT>
-__device__ __forceinline__ void xg_load(XStage<CT> &st, rsrc_t xr, int M, int K, int sb) {
-    const uint32_t so = uni(sb < 0 ? kNoLoad : (uint32_t)sb * 512u);
-#pragma unroll
-    for (int i = 0; i < 2 * CT; i++) {
-        const int piece = (int)threadIdx.x + 256 * i, r = piece >> 5, col = piece & 31;
-        const uint32_t vo = r < M ? (uint32_t)r * (uint32_t)K * 2u + (uint32_t)col * 16u : kNoLoad;
-        st.v[i] = bld16(xr, vo, so);
-    }
-}
-template <int CT> __device__ __forceinline__ void xg_store(const XStage<CT> &st, uint8_t *buf) {
-#pragma unroll
-    for (int i = 0; i < 2 * CT; i++) {
-        const int piece = (int)threadIdx.x + 256 * i, r = piece >> 5, col = piece & 31;
-        *(uintx4 *)(buf + r * XG_PITCH + col * 16) = st.v[i];
-    }
-}
-
-template <int FMT, int RW, int CT>
-__device__ __forceinline__ void qgx_step(const typename QFmt<FMT>::D (&w)[RW], const uint8_t *xb,
-                                         const uint32_t (&boff)[CT], int g, floatx4 (&acc)[RW][CT]) {
-    typedef QFmt<FMT> F;
-    typename F::S sc[RW];
-#pragma unroll
-    for (int rt = 0; rt < RW; rt++) sc[rt] = F::scales(w[rt], g);
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-        half8 b[CT];
-#pragma unroll
-        for (int ct = 0; ct < CT; ct++) b[ct] = *(const half8 *)(xb + boff[ct] + 64 * c);
-#pragma unroll
-        for (int rt = 0; rt < RW; rt++) {
-            const half8 a = F::frag(w[rt], sc[rt], g, c);
-#pragma unroll
-            for (int ct = 0; ct < CT; ct++)
-                acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[ct], acc[rt][ct], 0, 0, 0);
-        }
-    }
-}
-
-// superblocks [sb0, sb1); every thread stages, waves with live = false only
-// keep the barriers
-template <int FMT, int RW, int CT>
-__device__ __forceinline__ void qgx_body(const GemmParams &p, const WRow (&row)[RW], bool live, int sb0, int sb1,
-                                         floatx4 (&acc)[RW][CT], uint8_t *lds) {
-    typedef QFmt<FMT> F;
-    const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
-    const int nsb = p.K >> 8;
-    constexpr int STAGE = CT * 16 * XG_PITCH;
-    const rsrc_t xr = make_rsrc(p.xp, (uint32_t)p.M * (uint32_t)p.K * 2u);
-    uint32_t boff[CT];
-#pragma unroll
-    for (int ct = 0; ct < CT; ct++) boff[ct] = (uint32_t)min(ct * 16 + r16, p.M - 1) * XG_PITCH + 16u * g;
-    typename F::D w0[RW], w1[RW];
-    XStage<CT> xs;
-    auto wsb = [&](int sb) { return live && sb < sb1 ? sb : -1; };
-    xg_load<CT>(xs, xr, p.M, p.K, sb0);
-#pragma unroll
-    for (int rt = 0; rt < RW; rt++) F::load(w0[rt], row[rt], nsb, wsb(sb0), g);
-    xg_store<CT>(xs, lds);
-    __syncthreads();
-    for (int sb = sb0;; sb += 2) {
-        // next superblock: activations first (the LDS store below waits on
-        // them only), then weights
-        xg_load<CT>(xs, xr, p.M, p.K, sb + 1 < sb1 ? sb + 1 : -1);
-#pragma unroll
-        for (int rt = 0; rt < RW; rt++) F::load(w1[rt], row[rt], nsb, wsb(sb + 1), g);
-        if (live) qgx_step<FMT, RW, CT>(w0, lds, boff, g, acc);
-        if (sb + 1 >= sb1) break;
-        xg_store<CT>(xs, lds + STAGE);
-        __syncthreads();
-        xg_load<CT>(xs, xr, p.M, p.K, sb + 2 < sb1 ? sb + 2 : -1);
-#pragma unroll
-        for (int rt = 0; rt < RW; rt++) F::load(w0[rt], row[rt], nsb, wsb(sb + 2), g);
-        if (live) qgx_step<FMT, RW, CT>(w1, lds + STAGE, boff, g, acc);
-        if (sb + 2 >= sb1) break;
-        xg_store<CT>(xs, lds);
-        __syncthreads();
-    }
-}
-
-template <int RW, int CT>
-__global__ __launch_bounds__(256) void k_qgx(GemmParams p, int nks) {
-    warm_kernargs<sizeof(GemmParams)>();
-    extern __shared__ __attribute__((aligned(16))) uint8_t xlds[];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r16 = lane & 15, g = lane >> 4;
-    const int rb = (int)blockIdx.x / nks, ks = (int)blockIdx.x % nks;
-    const bool swi = p.mode == GM_SWIGLU;
-    const int nfeat = swi ? p.seg[0].rows / 16 : 0;
-    // this wave's row tiles and their place among the launch's output rows
-    GemmSeg S[RW];
-    int rloc[RW], grow[RW];
-    bool live;
-    if (swi) {
-        const int f = rb * XG_WAVES + wave;
-        live = f < nfeat;
-#pragma unroll
-        for (int rt = 0; rt < RW; rt++) {
-            S[rt] = rt == 0 ? p.seg[0] : p.seg[1];
-            rloc[rt] = (live ? f : 0) * 16;
-            grow[rt] = rt * nfeat * 16 + rloc[rt];
-        }
-    } else {
-        const int t0 = (rb * XG_WAVES + wave) * RW;
-        live = t0 < p.ntiles;
-        const GemmSeg s = seg_of_tile(p, live ? t0 : 0);
-#pragma unroll
-        for (int rt = 0; rt < RW; rt++) {
-            S[rt] = s;
-            rloc[rt] = ((live ? t0 : s.tile0) - s.tile0 + rt) * 16;
-            grow[rt] = (live ? t0 : 0) * 16 + rt * 16;
-        }
-    }
-    WRow row[RW];
-#pragma unroll
-    for (int rt = 0; rt < RW; rt++) row[rt] = wrow(S[rt], p.K, rloc[rt]);
-    const int nsb = p.K >> 8;
-    const int sb0 = ks * nsb / nks, sb1 = (ks + 1) * nsb / nks;
-    // Input norm (norm_ssq set, M <= 64, norm_parts <= 64): thread t sums the
-    // partials j = t % 4, t % 4 + 4, ... of token t / 4, requested now and
-    // added after the main loop (norm_inv_rms's order)
-    const bool has_norm = p.norm_ssq != nullptr;
-    float nrm[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) nrm[i] = 0.f;
-    if (has_norm) {
-        const int m = min((int)threadIdx.x >> 2, p.M - 1), j0 = (int)threadIdx.x & 3;
-        const rsrc_t nr = make_rsrc(p.norm_ssq, (uint32_t)(p.M * p.norm_parts * 4));
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int j = j0 + 4 * i;
-            nrm[i] = __uint_as_float(bld4(nr, j < p.norm_parts ? (uint32_t)(m * p.norm_parts + j) * 4u : kNoLoad, 0u));
-        }
-    }
-    floatx4 acc[RW][CT];
-#pragma unroll
-    for (int rt = 0; rt < RW; rt++)
-#pragma unroll
-        for (int ct = 0; ct < CT; ct++) acc[rt][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
-    switch (S[0].fmt) {
-    case Q4_K: qgx_body<Q4_K, RW, CT>(p, row, live, sb0, sb1, acc, xlds); break;
-    case Q5_K: qgx_body<Q5_K, RW, CT>(p, row, live, sb0, sb1, acc, xlds); break;
-    case Q6_K: qgx_body<Q6_K, RW, CT>(p, row, live, sb0, sb1, acc, xlds); break;
-    case Q8_0: qgx_body<Q8_0, RW, CT>(p, row, live, sb0, sb1, acc, xlds); break;
-    default: break;
-    }
-    // 1 / rms of every token
-    __shared__ float s_inv[64];
-    if (has_norm) {
-        float t = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; i++) t += nrm[i];
-        t += __shfl_xor(t, 1);
-        t += __shfl_xor(t, 2);
-        if ((threadIdx.x & 3) == 0 && (int)(threadIdx.x >> 2) < p.M)
-            s_inv[threadIdx.x >> 2] = 1.0f / sqrtf(t / (float)p.K + p.norm_eps);
-        __syncthreads();
-    }
-    const int slot = rb * XG_WAVES + wave;  // argmax partial slot of this wave
-    if (!live) {
-        // padding waves of the last row block leave a neutral argmax partial
-        if (p.mode == GM_LOGITS && g == 0)
-            for (int m = r16; m < p.M; m += 16) {
-                p.amax_v[(int64_t)m * p.amax_ld + slot] = -INFINITY;
-                p.amax_i[(int64_t)m * p.amax_ld + slot] = 0x7fffffff;
-            }
-        if (nks == 1) return;
-    }
-    if (nks == 1) {
-#pragma unroll
-        for (int ct = 0; ct < CT; ct++) {
-            floatx4 v[RW];
-#pragma unroll
-            for (int rt = 0; rt < RW; rt++) v[rt] = acc[rt][ct];
-            if (has_norm) {
-                const float inv = s_inv[min(ct * 16 + r16, 63)];
-#pragma unroll
-                for (int rt = 0; rt < RW; rt++) v[rt] *= inv;
-            }
-            EpiPre<RW> e;
-            epi_prefetch<RW>(p, S, rloc, ct * 16 + r16, g, e);
-            epilogue<RW>(p, S, rloc, v, e, ct * 16 + r16, g, slot);
-        }
-        return;
-    }
-    // K slices: partial sums [ks][M][R] (R = output rows of the launch); the
-    // consumer of the output adds them in slice order (an in-kernel reduction
-    // by the last workgroup needs agent-scope fences, i.e. L2 write-back and
-    // invalidation on every XCD, which measured slower than the split saved)
-    if (!live) return;
-    const int R = p.ntiles * 16;
-#pragma unroll
-    for (int ct = 0; ct < CT; ct++) {
-        const int m = ct * 16 + r16;
-        if (m >= p.M) continue;
-#pragma unroll
-        for (int rt = 0; rt < RW; rt++)
-            *(floatx4 *)(p.part + ((int64_t)ks * p.M + m) * R + grow[rt] + 4 * g) = acc[rt][ct];
-    }
-}
-
 // --------------------------------------------------------------------------
 // Launch policy.  KW (waves splitting K) is a function of the matrix only --
 // the smallest power of two that reaches the policy's wave count, capped at 8
@@ -1173,13 +907,11 @@ int qgemm_kw(const GemmParams &p) {
     return kw;
 }
 
-static int token_tiles(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8; }
-
-// Row tiles of a wave: the policy's for up to two token tiles, else 1 (gate/up
-// pairs always 2); shrunk until every segment splits evenly.
+// Row tiles of a wave: the policy's, shrunk until every segment splits evenly
+// (gate/up pairs always 2).
 static int qgemm_rt(const GemmParams &p) {
     if (p.mode == GM_SWIGLU) return 2;
-    int rt = token_tiles(p.M) <= 2 ? policy_rt(p) : 1;
+    int rt = policy_rt(p);
     for (; rt > 1; rt /= 2) {
         bool ok = p.ntiles % rt == 0;
         for (int i = 0; i < p.nseg; i++) ok = ok && (p.seg[i].rows / 16) % rt == 0;
@@ -1188,32 +920,10 @@ static int qgemm_rt(const GemmParams &p) {
     return rt;
 }
 
-// ---- M > 16: row blocks of 4 waves, K slices towards one workgroup per CU ----
-static int xg_rw(const GemmParams &p) {
-    if (p.mode == GM_SWIGLU) return 2;
-    if (token_tiles(p.M) > 4) return 1;
-    for (int i = 0; i < p.nseg; i++)
-        if ((p.seg[i].rows / 16) % 2) return 1;
-    return 2;
-}
-static int xg_row_blocks(const GemmParams &p) {
-    const int units = p.mode == GM_SWIGLU ? swiglu_features(p) : p.ntiles / xg_rw(p);
-    return (units + XG_WAVES - 1) / XG_WAVES;
-}
-// K slices: only when the caller finalises them (allow_split), towards 192
-// workgroups, up to 8 slices and the partial-sum buffer
-int qgemm_slices(const GemmParams &p) {
-    if (p.M <= 16 || !p.allow_split || (p.mode != GM_STORE && p.mode != GM_RESID)) return 1;
-    const int rb = xg_row_blocks(p), nsb = p.K / 256;
-    const int64_t R = 16LL * p.ntiles;
-    int ks = 1;
-    while (ks < 8 && rb * ks < 192 && 2 * ks <= nsb && (int64_t)2 * ks * p.M * R <= p.part_cap) ks *= 2;
-    return ks;
-}
-
 // argmax partial slots of a GM_LOGITS launch (= amax_ld)
+int qgemm_slices(const GemmParams &p) { return p.M > 16 ? qwide_slices(p) : 1; }
 int qgemm_workgroups(const GemmParams &p) {
-    if (p.M > 16) return xg_row_blocks(p) * XG_WAVES;
+    if (p.M > 16) return qwide_slots(p);
     const int rt = qgemm_rt(p);
     return p.mode == GM_SWIGLU ? swiglu_features(p) / (rt / 2) : p.ntiles / rt;
 }
@@ -1223,13 +933,6 @@ static void launch_timed(Kern kern, dim3 grid, dim3 block, size_t lds, hipStream
                          Args... args) {
     if (tm.start && tm.stop) hipExtLaunchKernelGGL(kern, grid, block, lds, st, tm.start, tm.stop, 0, args...);
     else hipLaunchKernelGGL(kern, grid, block, lds, st, args...);
-}
-
-template <int RW, int CT>
-static void launch_qgx(const GemmParams &p, hipStream_t st, const LaunchTiming &tm) {
-    const int rb = xg_row_blocks(p), nks = qgemm_slices(p);
-    const size_t lds = 2 * CT * 16 * XG_PITCH;
-    launch_timed(k_qgx<RW, CT>, dim3(rb * nks), dim3(64 * XG_WAVES), lds, st, tm, p, nks);
 }
 
 template <int RT, int KW>
@@ -1323,16 +1026,8 @@ void launch_qkv_attention(const GemmParams &g, const AttnParams &a, const QkvAtt
 
 int launch_qgemm(const GemmParams &p, hipStream_t st, const LaunchTiming &tm) {
     qgemm_check(p);
-    const int ct = token_tiles(p.M);
-    if (ct > 1) {
-        if (qgemm_slices(p) > 1 && !p.part) throw BackendError("qgemm: split-K workspace missing");
-        const int rw = xg_rw(p);
-        if (rw == 2 && ct == 2) launch_qgx<2, 2>(p, st, tm);
-        else if (rw == 2 && ct == 4) launch_qgx<2, 4>(p, st, tm);
-        else if (rw == 2 && ct == 8) launch_qgx<2, 8>(p, st, tm);
-        else if (rw == 1 && ct == 2) launch_qgx<1, 2>(p, st, tm);
-        else if (rw == 1 && ct == 4) launch_qgx<1, 4>(p, st, tm);
-        else launch_qgx<1, 8>(p, st, tm);
+    if (p.M > 16) {
+        launch_qwide(p, st, tm);
         return qgemm_workgroups(p);
     }
     const int kw = qgemm_kw(p), rt = qgemm_rt(p);
