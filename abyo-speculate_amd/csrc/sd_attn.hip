@@ -241,7 +241,7 @@ __device__ __forceinline__ void tile_store(uintx4 *stage, const TileCopy<HD> &c,
 
 // One 32-key block from LDS for the wave's query tiles (dead tiles skipped)
 // (lp: the lane's swizzled piece inside a chunk, lds_swz(r16 * 4 + g))
-template <int HD, int QT>
+template <int HD, int QT, bool CAUSAL>
 __device__ __forceinline__ void tile_step(AttnState<HD, QT> &S, const uintx4 *stage, int lp, const bool (&tl)[QT],
                                           int kk, int P, int T, int lim, int g) {
     constexpr int NDC = HD / 32, NDT = HD / 16;
@@ -260,7 +260,7 @@ __device__ __forceinline__ void tile_step(AttnState<HD, QT> &S, const uintx4 *st
         if (!tl[t]) continue;
         floatx4 st[2];
         step_scores<HD, QT>(S, kop, t, st);
-        bp[t] = step_softmax<HD, QT>(S, t, st, kk, P, T, lim, g, alpha[t], moved);
+        bp[t] = step_softmax<HD, QT, CAUSAL>(S, t, st, kk, P, T, lim, g, alpha[t], moved);
     }
     uintx4 vop[NDT];
 #pragma unroll
@@ -271,17 +271,20 @@ __device__ __forceinline__ void tile_step(AttnState<HD, QT> &S, const uintx4 *st
 
 template <int HD> constexpr size_t attn_t_lds() { return (size_t)kTStages * 8 * HD * 16; }
 
-template <int HD>
+// CAUSAL: a prompt's rows.  A query block stops at its last row's last key (so
+// does a wave's tile), and the heaviest blocks, the last, start first.
+template <int HD, bool CAUSAL>
 __global__ __launch_bounds__(kTThreads) void k_attn_t(AttnParams p) {
     warm_kernargs<sizeof(AttnParams)>();
     constexpr int QT = kTQW, SW = 8 * HD;  // SW: 16-byte pieces of one stage
     extern __shared__ uintx4 lds[];
-    const int h = blockIdx.x, s = blockIdx.y, qb = blockIdx.z;
+    const int h = blockIdx.x, s = blockIdx.y, qb = CAUSAL ? (int)(gridDim.z - 1 - blockIdx.z) : (int)blockIdx.z;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tid = threadIdx.x;
     const int r16 = lane & 15, g = lane >> 4;
     const int nq = p.M * p.n_rep;
-    const int T = p.P + p.M;
+    // keys past T hold stale rows; a causal query block needs none past its last row's
+    const int T = p.P + (CAUSAL ? min(p.M, (min((qb + 1) * kTWaves * kTQW * 16, nq) - 1) / p.n_rep + 1) : p.M);
     const int kps = 4 * p.keys_per_wave;  // keys of a split
     const int k0 = s * kps, lim = min(k0 + kps, T);
     const int nb = (lim - k0 + 31) / 32;
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(kTThreads) void k_attn_t(AttnParams p) {
     for (int t = 0; t < QT; t++) {
         const int tile = (qb * kTWaves + wave) * QT + t;
         tl[t] = tile * 16 < nq;  // wave-uniform: the tile holds a live query
-        query_fetch<HD>(qr[t], p, h, tile * 16 + r16, g);
+        query_fetch<HD, false, CAUSAL>(qr[t], p, h, tile * 16 + r16, g);
     }
     TileCopy<HD> c0, c1, c2;
     tile_fetch<HD>(c0, src, blk(0), tid);
@@ -312,23 +315,30 @@ __global__ __launch_bounds__(kTThreads) void k_attn_t(AttnParams p) {
 #pragma unroll
     for (int t = 0; t < QT; t++) query_init<HD, QT>(S, t, qr[t], sl2);
 
+    // keys below Pv are visible to every query of the wave, keys from Pe on to none
+    const int Pv = CAUSAL ? p.P + min((qb * kTWaves + wave) * QT * 16, nq - 1) / p.n_rep + 1 : p.P;
+    const int Pe = CAUSAL ? p.P + (min(((qb * kTWaves + wave) * QT + QT) * 16, nq) - 1) / p.n_rep + 1 : T;
+    auto tstep = [&](const uintx4 *stage, int kk) {
+        if (!CAUSAL || kk < Pe) tile_step<HD, QT, CAUSAL>(S, stage, lp, tl, kk, Pv, T, lim, g);
+    };
+
     // block j lives in stage j % 3; it is written after every wave passed the
     // barrier of block j - 1, i.e. finished block j - 2 and so block j - 3.
     for (int j = 0; j < nb; j += 3) {
         tile_store<HD>(lds, c0, tid);
         tile_fetch<HD>(c0, src, blk(j + 3), tid);
         __syncthreads();
-        tile_step<HD, QT>(S, lds, lp, tl, k0 + 32 * j, p.P, T, lim, g);
+        tstep(lds, k0 + 32 * j);
         if (j + 1 >= nb) break;
         tile_store<HD>(lds + SW, c1, tid);
         tile_fetch<HD>(c1, src, blk(j + 4), tid);
         __syncthreads();
-        tile_step<HD, QT>(S, lds + SW, lp, tl, k0 + 32 * (j + 1), p.P, T, lim, g);
+        tstep(lds + SW, k0 + 32 * (j + 1));
         if (j + 2 >= nb) break;
         tile_store<HD>(lds + 2 * SW, c2, tid);
         tile_fetch<HD>(c2, src, blk(j + 5), tid);
         __syncthreads();
-        tile_step<HD, QT>(S, lds + 2 * SW, lp, tl, k0 + 32 * (j + 2), p.P, T, lim, g);
+        tstep(lds + 2 * SW, k0 + 32 * (j + 2));
     }
 #pragma unroll
     for (int t = 0; t < QT; t++) {
@@ -446,6 +456,15 @@ AttnSplit attn_split(int P, int M, int n_kv, int n_rep) {
     return AttnSplit{32 * spw, (T + kps - 1) / kps};
 }
 
+// k_attn_t over a prompt's rows: query blocks first, and where they leave CUs
+// idle, as many splits as fill them
+AttnSplit attn_split_causal(int P, int M, int n_kv, int n_rep, int max_splits) {
+    const int T = P + M, nqt = (M * n_rep + 15) / 16, nqb = (nqt + kTWaves * kTQW - 1) / (kTWaves * kTQW);
+    const int want = std::max(1, std::min(max_splits, 256 / (n_kv * nqb)));
+    const int kps = ((T + want - 1) / want + 31) / 32 * 32;
+    return AttnSplit{kps / 4, (T + kps - 1) / kps};
+}
+
 // above 16 rows the split size is >= (P + 1) / want and >= 32 with
 // want <= kTMaxSplits, so for M <= 128 nsplit = ceil((P + M) / size) <=
 // want + 1 + 128 / 32; up to 16 rows a split holds 768 keys below 1024
@@ -464,10 +483,13 @@ static void allow_attn_t_lds() {
     SD_ATTN_CHECK(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lock(mu);
     if ((size_t)dev < done.size() && done[dev]) return;
-    SD_ATTN_CHECK(hipFuncSetAttribute((const void *)k_attn_t<128>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)attn_t_lds<128>()));
-    SD_ATTN_CHECK(hipFuncSetAttribute((const void *)k_attn_t<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)attn_t_lds<64>()));
+    const auto set = [](const void *f, size_t lds) {
+        SD_ATTN_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    };
+    set((const void *)k_attn_t<128, false>, attn_t_lds<128>());
+    set((const void *)k_attn_t<64, false>, attn_t_lds<64>());
+    set((const void *)k_attn_t<128, true>, attn_t_lds<128>());
+    set((const void *)k_attn_t<64, true>, attn_t_lds<64>());
     if ((size_t)dev >= done.size()) done.resize(dev + 1, false);
     done[dev] = true;
 }
@@ -481,7 +503,8 @@ static void attn_check(const AttnParams &p) {
     if ((int64_t)(p.nsplit - 1) * waves * p.keys_per_wave >= (int64_t)p.P + p.M)
         throw BackendError("attention: empty split");
     if (p.cap % 32 || (int64_t)p.P + p.M > p.cap) throw BackendError("attention: cache capacity");
-    if (p.mask_words < 1 || p.mask_words > 2 || p.M > 64 * p.mask_words) throw BackendError("attention: mask words");
+    if (p.mask_words == 0 && p.M <= 16) throw BackendError("attention: causal rows without masks need more than 16");
+    if (p.mask_words != 0 && (p.mask_words < 1 || p.mask_words > 2 || p.M > 64 * p.mask_words)) throw BackendError("attention: mask words");
     if (p.hd != 128 && p.hd != 64) throw BackendError("attention: head_dim must be 64 or 128");
 }
 
@@ -522,8 +545,11 @@ void launch_attention(const AttnParams &p, hipStream_t st) {
         const int nqt = (p.M * p.n_rep + 15) / 16;
         const dim3 grid(p.n_kv, p.nsplit, (nqt + kTWaves * kTQW - 1) / (kTWaves * kTQW));
         allow_attn_t_lds();
-        if (p.hd == 128) hipLaunchKernelGGL(k_attn_t<128>, grid, dim3(kTThreads), attn_t_lds<128>(), st, p);
-        else hipLaunchKernelGGL(k_attn_t<64>, grid, dim3(kTThreads), attn_t_lds<64>(), st, p);
+        const bool causal = p.mask_words == 0;
+        if (p.hd == 128 && causal) hipLaunchKernelGGL((k_attn_t<128, true>), grid, dim3(kTThreads), attn_t_lds<128>(), st, p);
+        else if (p.hd == 128) hipLaunchKernelGGL((k_attn_t<128, false>), grid, dim3(kTThreads), attn_t_lds<128>(), st, p);
+        else if (causal) hipLaunchKernelGGL((k_attn_t<64, true>), grid, dim3(kTThreads), attn_t_lds<64>(), st, p);
+        else hipLaunchKernelGGL((k_attn_t<64, false>), grid, dim3(kTThreads), attn_t_lds<64>(), st, p);
         launch_attn_combine(p, st);
         return;
     }

@@ -104,7 +104,8 @@ template <int HD> struct QueryRaw {
 };
 // DEV: the queries were written during this launch by other workgroups and
 // are read at device scope.
-template <int HD, bool DEV = false>
+// CAUSAL: mk0 is the row's last visible key.
+template <int HD, bool DEV = false, bool CAUSAL = false>
 __device__ __forceinline__ void query_fetch(QueryRaw<HD> &r, const AttnParams &p, int h, int q, int g) {
     const int nq = p.M * p.n_rep;
     r.live = q < nq;
@@ -119,6 +120,11 @@ __device__ __forceinline__ void query_fetch(QueryRaw<HD> &r, const AttnParams &p
         } else {
             r.q[dc] = *(const uintx4 *)(qr + dc * 32 + g * 8);
         }
+    }
+    if constexpr (CAUSAL) {
+        r.mk0 = (uint64_t)(p.P + m);
+        r.mk1 = 0ull;
+        return;
     }
     r.mk0 = p.mask[(int64_t)m * p.mask_words];
     r.mk1 = p.mask_words > 1 ? p.mask[(int64_t)m * p.mask_words + 1] : 0ull;
@@ -153,7 +159,8 @@ __device__ __forceinline__ void query_init(AttnState<HD, QT> &S, int t, const Qu
 // traffic at all: the max is only gathered (and the accumulators rescaled by
 // alpha) when some lane of the wave sees a score above its m + 8.
 // Keys at or past lim (<= T) belong to another range and are masked.
-template <int HD, int QT>
+// CAUSAL: every query sees the keys below P, and those up to its own mk0.
+template <int HD, int QT, bool CAUSAL = false>
 __device__ __forceinline__ half8 step_softmax(AttnState<HD, QT> &S, int t, floatx4 (&st)[2], int kk, int P, int T,
                                               int lim, int g, float &alpha, bool &moved) {
     const bool full = kk + 32 <= P && kk + 32 <= lim;  // every key of the step is visible to every query
@@ -166,7 +173,9 @@ __device__ __forceinline__ half8 step_softmax(AttnState<HD, QT> &S, int t, float
             if (!full) {
                 const int key = kk + kt * 16 + 4 * g + i;
                 bool vis = key < P && key < lim;
-                if (!vis && key < lim) {
+                if constexpr (CAUSAL) {
+                    vis = key <= (int)S.mk0[t] && key < lim;
+                } else if (!vis && key < lim) {
                     const int tt = key - P;
                     vis = (((tt < 64 ? S.mk0[t] : S.mk1[t]) >> (tt & 63)) & 1ull) != 0;
                 }

@@ -13,17 +13,17 @@ namespace sd {
 
 #pragma clang fp contract(off)
 
-// One workgroup (NT threads) per row.  Each thread keeps its K/NT values in
+// One workgroup per row (K / (4 NV) threads).  Each thread keeps its 4 NV values in
 // registers (vector loads, all issued before the first use), so the row is
-// read from memory once and there is one memory round trip, not K/NT of them.
+// read from memory once and there is one memory round trip, not one per value.
 // With nks > 1 the residual matmul that produced x left K-slice partial sums
 // part[ks][M][K] (nks <= 8): they are added to x in slice order first (and x
 // is stored); every slice's loads are in flight before the first add.
-template <int NV, int NT>  // NT threads, NV float4 vectors per thread: K = 4 * NT * NV
-__global__ __launch_bounds__(NT) void k_rmsnorm(float *x, const float *w, int K, float eps, uint16_t *out16,
+template <int NV>  // NV float4 vectors per thread: K = 4 * NV * blockDim.x
+__global__ __launch_bounds__(1024) void k_rmsnorm(float *x, const float *w, int K, float eps, uint16_t *out16,
                                                 int ld16, float *out32, const float *part, int nks,
                                                 int64_t pstride, int tiled) {
-    const int m = blockIdx.x, t = threadIdx.x;
+    const int m = blockIdx.x, t = threadIdx.x, NT = blockDim.x;
     float4 *row = (float4 *)(x + (int64_t)m * K);
     const float4 *wv = (const float4 *)w;
     float4 v[NV], wr[NV];
@@ -64,13 +64,11 @@ __global__ __launch_bounds__(NT) void k_rmsnorm(float *x, const float *w, int K,
     ss += __shfl_xor(ss, 8);
     ss += __shfl_xor(ss, 16);
     ss += __shfl_xor(ss, 32);
-    constexpr int NW = NT / 64;
-    __shared__ float red[NW];
+    __shared__ float red[16];
     if ((t & 63) == 0) red[t >> 6] = ss;
     __syncthreads();
     float tot = 0.f;
-#pragma unroll
-    for (int i = 0; i < NW; i++) tot += red[i];  // fixed order
+    for (int i = 0; i < NT / 64; i++) tot += red[i];  // fixed order
     const float mrms = sqrtf(tot / (float)K + eps);
 #pragma unroll
     for (int i = 0; i < NV; i++) {
@@ -306,17 +304,13 @@ __global__ __launch_bounds__(256) void k_keep_kv_tail(uint16_t *kv, int64_t stre
 void launch_rmsnorm(float *x, const float *w, int M, int K, float eps, uint16_t *out16, int ld16, float *out32,
                     hipStream_t st, const float *part, int nks, int64_t ps, int tiled) {
 #define SD_RMS(KERN, NT) hipLaunchKernelGGL(KERN, dim3(M), dim3(NT), 0, st, x, w, K, eps, out16, ld16, out32, part, nks, ps, tiled)
-    // one float4 per thread (and slice) where K allows: the row's loads spread
-    // over 16 waves
-    switch (K) {
-    case 1024: SD_RMS((k_rmsnorm<1, 256>), 256); break;
-    case 2048: SD_RMS((k_rmsnorm<2, 256>), 256); break;
-    case 3072: SD_RMS((k_rmsnorm<3, 256>), 256); break;
-    case 4096: SD_RMS((k_rmsnorm<1, 1024>), 1024); break;
-    case 5120: SD_RMS((k_rmsnorm<5, 256>), 256); break;
-    case 8192: SD_RMS((k_rmsnorm<2, 1024>), 1024); break;
-    default: SD_RMS(k_rmsnorm_any, 256); break;
-    }
+    // as few float4 per thread (and slice) as 1024 threads allow: the row's
+    // loads spread over the most waves.  K = 3584 took 20.4 us for 128 rows in
+    // the strided loop (a chain of scalar loads), 5 us here, as K = 4096.
+    if (K % 256 == 0 && K <= 4096) SD_RMS(k_rmsnorm<1>, K / 4);
+    else if (K % 512 == 0 && K <= 8192) SD_RMS(k_rmsnorm<2>, K / 8);
+    else if (K % 1024 == 0 && K <= 16384) SD_RMS(k_rmsnorm<4>, K / 16);
+    else SD_RMS(k_rmsnorm_any, 256);
 #undef SD_RMS
 }
 void launch_norm_u(const float *x, const float *w, int M, int K, uint16_t *out16, int ld16, float *ssq,

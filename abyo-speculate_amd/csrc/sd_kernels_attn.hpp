@@ -36,13 +36,15 @@ struct AttnSplit {
 };
 AttnSplit attn_split(int P, int M, int n_kv, int n_rep);
 int attn_max_splits(int n_kv);  // upper bound of nsplit over all P, M <= 128
+// the split of a prompt's M > 16 causal rows, at most max_splits
+AttnSplit attn_split_causal(int P, int M, int n_kv, int n_rep, int max_splits);
 
 struct AttnParams {
     const uint16_t *q16;
     const uint16_t *kc, *vc;
     int64_t cap;
     const uint64_t *mask;  // [M][mask_words]
-    int mask_words;
+    int mask_words;        // 0: causal (a prompt's rows: row m sees keys up to P + m), more than 16 rows
     int P, M, n_heads, n_kv, n_rep, hd;
     int keys_per_wave, nsplit;
     float scale;           // 1/sqrt(hd)

@@ -80,10 +80,11 @@ Model::~Model() {
                     (void *)acc_m, (void *)acc_s, (void *)acc_q, (void *)acc_am, (void *)acc_tree,
                     (void *)acc_out, (void *)t2d_inv, (void *)qg_part, (void *)aux_h, (void *)aux_x, (void *)aux_y,
                     (void *)aux_ids, (void *)ssq, (void *)split_cnt, (void *)acc_part, (void *)acc_cnt,
-                    (void *)acc_prob, (void *)acc_lin, (void *)qa_flags})
+                    (void *)acc_prob, (void *)acc_lin, (void *)qa_flags, (void *)d_prompt})
         F(p);
     if (qa_status) hipHostFree(qa_status);
     if (h_stage) hipHostFree(h_stage);
+    if (h_prompt) hipHostFree(h_prompt);
     if (acc_stage) hipHostFree(acc_stage);
     if (stage_ev) hipEventDestroy(stage_ev);
     for (hipEvent_t e : ev_pool) hipEventDestroy(e);
@@ -92,7 +93,16 @@ Model::~Model() {
 
 void Model::alloc_buffers() {
     const ModelCfg &c = cfg;
-    const int Mx = c.max_batch, Mp = 128 + 16;  // padded rows (16-token MFMA tiles + last-row slack)
+    const int Mx = c.max_batch;
+    // A prompt goes through the layers in chunks of up to kPromptRows rows (as
+    // many as the context holds), not max_batch: every chunk reads and
+    // dequantises all weights and pays the launches, and 128 rows leave the
+    // 4096-row matrices with 32 of 256 CUs' worth of tiles.  Above 2048 rows
+    // every matrix fills the chip, so more only costs memory (about 0.2 GB at
+    // the 8B shapes).
+    prompt_rows = std::max(Mx, std::min(kPromptRows, (c.ctx_len + 31) / 32 * 32));
+    // rows of the matmuls' inputs: whole 32-token tiles (and 16-token ones + slack)
+    const int Rp = prompt_rows, Mp = std::max(128 + 16, (Rp + 31) / 32 * 32);
     cap = ((int64_t)c.ctx_len + 128 + 31) / 32 * 32;  // whole 32-position blocks of the V layout
     kv = dalloc<uint16_t>((size_t)c.n_layers * 2 * c.n_kv_heads * cap * c.head_dim);
     // RoPE tables (quantized_llama_local.rs:189-205): host f32 powf/cosf/sinf
@@ -115,15 +125,16 @@ void Model::alloc_buffers() {
     xp_ld = std::max(c.hidden, c.q_dim());
     ap_ld = c.q_dim();
     act_ld = c.ffn;
-    h = dalloc<float>((size_t)Mx * c.hidden);
-    qkv = dalloc<float>((size_t)Mx * qkvd);
+    h = dalloc<float>((size_t)Rp * c.hidden);
+    qkv = dalloc<float>((size_t)Rp * qkvd);
     xp = dalloc<uint16_t>((size_t)Mp * xp_ld);
     ap = dalloc<uint16_t>((size_t)Mp * ap_ld);
     act = dalloc<uint16_t>((size_t)Mp * act_ld);
-    q16 = dalloc<uint16_t>((size_t)c.n_heads * Mx * c.head_dim);
+    q16 = dalloc<uint16_t>((size_t)c.n_heads * Rp * c.head_dim);
     nsplit_max = attn_max_splits(c.n_kv_heads);
-    part_o = dalloc<float>((size_t)nsplit_max * c.n_heads * Mx * c.head_dim);
-    part_ml = dalloc<float>((size_t)nsplit_max * c.n_heads * Mx * 2);
+    part_rows = std::max<int64_t>((int64_t)nsplit_max * Mx, 2 * Rp);
+    part_o = dalloc<float>((size_t)part_rows * c.n_heads * c.head_dim);
+    part_ml = dalloc<float>((size_t)part_rows * c.n_heads * 2);
     split_cnt = dalloc<int>(c.n_heads);  // n_kv x (query tiles <= n_rep up to 16 rows), zero
     qa_flags = dalloc<unsigned>(kQaFlags);
     SD_HIP_CHECK(hipHostMalloc((void **)&qa_status, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
@@ -148,6 +159,7 @@ void Model::alloc_buffers() {
     d_pos = d_ids + Mx;
     d_mask = (uint64_t *)(d_ids + 3 * Mx + (Mx & 1));
     d_src = dalloc<int>(Mx);
+    d_prompt = dalloc<int>((size_t)2 * Rp);
     qg_part_cap = std::max<int64_t>((int64_t)8 * Mx * std::max(qkvd, c.hidden), (int64_t)2 * Mx * 2 * c.ffn);
     qg_part = dalloc<float>((size_t)qg_part_cap);
     ssq = dalloc<float>((size_t)16 * (c.hidden / 16));
@@ -166,6 +178,7 @@ void Model::alloc_buffers() {
     aux_ids = dalloc<int>(kAuxRows);
     h_stage_bytes = (size_t)Mx * (3 * sizeof(int) + 2 * sizeof(uint64_t)) + 256;
     SD_HIP_CHECK(hipHostMalloc((void **)&h_stage, h_stage_bytes, hipHostMallocDefault));
+    SD_HIP_CHECK(hipHostMalloc((void **)&h_prompt, (size_t)2 * Rp * sizeof(int), hipHostMallocDefault));
     SD_HIP_CHECK(hipHostMalloc((void **)&acc_stage, ((size_t)(kAccTreeInts + 1) * Mx + 8) * sizeof(int),
                                hipHostMallocDefault));
     SD_HIP_CHECK(hipEventCreateWithFlags(&stage_ev, hipEventDisableTiming));
@@ -584,9 +597,12 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
                     int logits_mode, bool want_hidden, const std::vector<int> &collect, float *collect_out) {
     fwd_count++;
     const ModelCfg &c = cfg;
-    if (M < 1 || M > c.max_batch) throw ArgError("forward: M out of range");
+    // a prompt's rows are causal and need neither masks nor an output per row
+    const bool prompt = mask_words == 0;
+    if (M < 1 || M > (prompt ? prompt_rows : c.max_batch)) throw ArgError("forward: M out of range");
+    if (prompt && (M <= 16 || logits_mode == 2 || !collect.empty())) throw ArgError("forward: prompt rows");
     if (P + M > c.ctx_len) throw ArgError("forward: KV capacity exceeded");
-    if (mask_words < 1 || mask_words > 2) throw ArgError("forward: mask words");
+    if (mask_words < 0 || mask_words > 2) throw ArgError("forward: mask words");
     SD_HIP_CHECK(hipSetDevice(c.device));
     check_status();  // a fused launch of an earlier forward that gave up
     // fault injection for tests (SD_ATTN_WAIT_TEST=<reads>): the fused
@@ -597,18 +613,30 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
     // stage ids | pos | mask in pinned memory with the device block's layout,
     // then one H2D copy
     stage_wait();
-    std::memcpy(h_stage, ids, M * sizeof(int));
-    std::memcpy(h_stage + c.max_batch, pos, M * sizeof(int));
-    const size_t mask_at = (size_t)3 * c.max_batch + (c.max_batch & 1);
-    std::memcpy(h_stage + mask_at, mask, (size_t)M * mask_words * sizeof(uint64_t));
-    SD_HIP_CHECK(hipMemcpyAsync(d_ids, h_stage, mask_at * sizeof(int) + (size_t)M * mask_words * sizeof(uint64_t),
-                                hipMemcpyHostToDevice, st));
+    const int *ids_dev = d_ids, *pos_dev = d_pos;
+    if (prompt) {
+        std::memcpy(h_prompt, ids, M * sizeof(int));
+        std::memcpy(h_prompt + M, pos, M * sizeof(int));
+        SD_HIP_CHECK(hipMemcpyAsync(d_prompt, h_prompt, (size_t)2 * M * sizeof(int), hipMemcpyHostToDevice, st));
+        ids_dev = d_prompt;
+        pos_dev = d_prompt + M;
+    } else {
+        std::memcpy(h_stage, ids, M * sizeof(int));
+        std::memcpy(h_stage + c.max_batch, pos, M * sizeof(int));
+        const size_t mask_at = (size_t)3 * c.max_batch + (c.max_batch & 1);
+        std::memcpy(h_stage + mask_at, mask, (size_t)M * mask_words * sizeof(uint64_t));
+        SD_HIP_CHECK(hipMemcpyAsync(d_ids, h_stage,
+                                    mask_at * sizeof(int) + (size_t)M * mask_words * sizeof(uint64_t),
+                                    hipMemcpyHostToDevice, st));
+    }
     stage_done();
 
     const int H = c.hidden, QD = c.q_dim(), KVD = c.kv_dim(), QKVD = QD + 2 * KVD;
-    launch_embed(gw[K_TOK_EMBD].fmt, embed_table(), H, d_ids, M, h, st);
-    const AttnSplit split = attn_split(P, M, c.n_kv_heads, c.n_heads / c.n_kv_heads);
-    if (split.nsplit > nsplit_max) throw BackendError("attention split count exceeds workspace");
+    launch_embed(gw[K_TOK_EMBD].fmt, embed_table(), H, ids_dev, M, h, st);
+    const int max_splits = (int)std::min<int64_t>(nsplit_max, part_rows / M);
+    const AttnSplit split = prompt ? attn_split_causal(P, M, c.n_kv_heads, c.n_heads / c.n_kv_heads, max_splits)
+                                   : attn_split(P, M, c.n_kv_heads, c.n_heads / c.n_kv_heads);
+    if (split.nsplit > max_splits) throw BackendError("attention split count exceeds workspace");
     // M > 16 matmuls may leave K-slice partial sums in qg_part for the next
     // kernel to add (rope for QKV, the following RMSNorm for the residual
     // matmuls); not while per-layer hidden states are collected
@@ -695,7 +723,7 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
                 p.norm_parts = np;
                 p.norm_eps = c.rms_eps;
                 RopeOut &R = p.rope;
-                R.pos = d_pos;
+                R.pos = pos_dev;
                 R.cos_t = cos_t;
                 R.sin_t = sin_t;
                 R.q16 = q16;
@@ -732,7 +760,7 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
             RopeKvParams r{};
             r.qkv = qkv;
             r.ld_qkv = QKVD;
-            r.pos = d_pos;
+            r.pos = pos_dev;
             r.cos_t = cos_t;
             r.sin_t = sin_t;
             r.q16 = q16;
@@ -1053,8 +1081,42 @@ void Decoder::truncate(size_t len) {
     cache_len = (int)len;
 }
 
+// One pass where n rows fit max_batch.  A longer input goes in prompt chunks
+// of up to prompt_rows, evenly sized, in place of max_batch: the weights are
+// read and dequantised once per chunk, not once per max_batch rows.  What is
+// left of n over max_batch stays a pass of its own where it has up to 16 rows
+// (those kernels use the K-quant weights exactly), and so do all passes of a
+// handle whose max_batch is up to 16.
+void Decoder::advance(const uint32_t *tokens, size_t n, int logits_mode, bool want_hidden) {
+    Model &m = *model;
+    const size_t mb = m.cfg.max_batch, tail = n % mb;
+    const size_t wide = n <= mb || mb <= 16 ? 0 : tail <= 16 ? n - tail : n;
+    std::vector<int> ids, pos;
+    std::vector<uint64_t> mw;
+    for (size_t done = 0; done < n;) {
+        int M, nw = 0;
+        if (done < wide) {
+            const size_t left = wide - done, chunks = (left + m.prompt_rows - 1) / m.prompt_rows;
+            M = (int)((left + chunks - 1) / chunks);
+        } else {
+            M = (int)std::min(mb, n - done);
+        }
+        const bool last = done + M == n;
+        ids.assign(tokens + done, tokens + done + M);
+        pos.resize(M);
+        for (int i = 0; i < M; i++) pos[i] = cache_len + i;
+        if (done < wide && M > (int)mb) mw.clear();
+        else causal_masks(M, mw, nw);
+        const bool keep = n == 1 && !collect_keep.empty();
+        m.forward(ids.data(), pos.data(), mw.data(), nw, M, cache_len, last ? logits_mode : 0, last && want_hidden,
+                  keep && !want_hidden ? collect_keep : std::vector<int>{}, nullptr);
+        cache_len += M;
+        done += M;
+    }
+}
+
 // forward_advance_logits (quantized_llama.rs:137-158): forward `tokens` at the
-// cache end; caches the last row's logits.  Chunks longer inputs by max_batch.
+// cache end; caches the last row's logits.
 void Decoder::forward_advance(const uint32_t *tokens, size_t n, bool all_rows) {
     if (n == 0) throw SamplingError("forward_advance with empty tokens");
     Model &m = *model;
@@ -1063,23 +1125,7 @@ void Decoder::forward_advance(const uint32_t *tokens, size_t n, bool all_rows) {
         if (tokens[i] >= (uint32_t)V) throw ArgError("token id out of range");
     if (all_rows && n > (size_t)m.cfg.max_batch) throw ArgError("too many rows for one verify pass");
     if (cache_len + n > (size_t)m.cfg.ctx_len) throw ArgError("KV capacity exceeded");
-    size_t done = 0;
-    std::vector<int> ids, pos;
-    std::vector<uint64_t> mw;
-    int nw;
-    while (done < n) {
-        const int M = (int)std::min<size_t>(m.cfg.max_batch, n - done);
-        const bool last_chunk = done + M == n;
-        ids.assign(tokens + done, tokens + done + M);
-        pos.resize(M);
-        for (int i = 0; i < M; i++) pos[i] = cache_len + i;
-        causal_masks(M, mw, nw);
-        const bool keep = n == 1 && !collect_keep.empty();
-        m.forward(ids.data(), pos.data(), mw.data(), nw, M, cache_len, last_chunk ? (all_rows ? 2 : 1) : 0, false,
-                  keep ? collect_keep : std::vector<int>{}, nullptr);
-        cache_len += M;
-        done += M;
-    }
+    advance(tokens, n, all_rows ? 2 : 1, false);
     const int rows = m.logits_rows_last;
     SD_HIP_CHECK(hipMemcpyAsync(m.last_row, m.logits + (size_t)(rows - 1) * V, (size_t)V * 4,
                                 hipMemcpyDeviceToDevice, m.st));
@@ -1246,20 +1292,7 @@ void Decoder::observe_returning_last_hidden(const uint32_t *ids, size_t n, float
     if (cache_len + n > (size_t)m.cfg.ctx_len) throw ArgError("KV capacity exceeded");
     for (size_t i = 0; i < n; i++)
         if (ids[i] >= (uint32_t)m.cfg.vocab) throw ArgError("token id out of range");
-    size_t done = 0;
-    std::vector<int> tk, pos;
-    std::vector<uint64_t> mw;
-    int nw;
-    while (done < n) {
-        const int M = (int)std::min<size_t>(m.cfg.max_batch, n - done);
-        tk.assign(ids + done, ids + done + M);
-        pos.resize(M);
-        for (int i = 0; i < M; i++) pos[i] = cache_len + i;
-        causal_masks(M, mw, nw);
-        m.forward(tk.data(), pos.data(), mw.data(), nw, M, cache_len, 0, done + M == n, {}, nullptr);
-        cache_len += M;
-        done += M;
-    }
+    advance(ids, n, 0, true);
     history.insert(history.end(), ids, ids + n);
     if (out)
         SD_HIP_CHECK(hipMemcpyAsync(out, m.hidden_out, (size_t)m.cfg.hidden * 4,

@@ -115,7 +115,8 @@ class Model {
     double bench_qmatmul(int layer, int kind, int M, int iters, double *bytes_out);
     GemmParams bench_params(int layer, int kind, int M, double *bytes_out);
 
-    // forward of M tokens at cache positions [P, P+M); mask words per token.
+    // forward of M tokens at cache positions [P, P+M); mask words per token (0:
+    // a prompt's causal rows, 17 to prompt_rows of them, no per-row outputs).
     // logits_mode: 0 none, 1 last row only (into logits row 0), 2 all rows.
     void forward(const int *ids, const int *pos, const uint64_t *mask, int mask_words, int M, int P, int logits_mode,
                  bool want_hidden, const std::vector<int> &collect, float *collect_out);
@@ -136,6 +137,10 @@ class Model {
     int prof_events();                             // index of a free (start, stop) event pair
     int prof_begin();                              // records a start event, returns its index
     void prof_end(int ev, int cls, double bytes);  // records the stop event
+
+    // Most rows of one forward of a prompt, at least max_batch.
+    static constexpr int kPromptRows = 2048;
+    int prompt_rows = 0;
 
     // device buffers
     uint16_t *kv = nullptr;  // [L][2][n_kv][cap][hd]
@@ -164,6 +169,7 @@ class Model {
     void check_status();
     int *amax_i = nullptr, *argmax = nullptr, *d_ids = nullptr, *d_pos = nullptr, *d_src = nullptr;
     uint64_t *d_mask = nullptr;
+    int *d_prompt = nullptr;  // a prompt's ids | positions [2][prompt_rows]
     // split-K partial sums of the M > 16 matmul (see GemmParams::allow_split)
     float *qg_part = nullptr;
     int64_t qg_part_cap = 0;
@@ -191,6 +197,7 @@ class Model {
     int xp_ld = 0, ap_ld = 0, act_ld = 0;
     int amax_ld = 0;
     int nsplit_max = 0;
+    int64_t part_rows = 0;     // (split, row) pairs of part_o, part_ml
     int logits_rows_last = 0;  // rows of `logits` / `argmax` produced by the last forward
     // apply_lm_head / embed_tokens work buffers (kAuxRows rows per chunk),
     // apart from the verify pass's
@@ -200,6 +207,7 @@ class Model {
     int *aux_ids = nullptr;
     // pinned staging for small H2D transfers
     int *h_stage = nullptr;
+    int *h_prompt = nullptr;
     int *acc_stage = nullptr;  // pinned: a walk's inputs [kAccTreeInts max_batch] and outputs [max_batch + 4]
     size_t h_stage_bytes = 0;
     hipEvent_t stage_ev = nullptr;  // recorded after the last copy out of h_stage
@@ -277,6 +285,8 @@ class Decoder {
 
   private:
     void forward_advance(const uint32_t *tokens, size_t n, bool all_rows);
+    // the forwards of n tokens at the cache end; the last one with these outputs
+    void advance(const uint32_t *tokens, size_t n, int logits_mode, bool want_hidden);
     // the acceptance walk over logits rows [0, n) of the last pass
     void accept_walk(const int *parents, const int *tokens, int n, const float *q_rows, bool q_on_device,
                      size_t q_rows_n, size_t q_vocab, const int *q_row_of, const float *uniforms, float temperature,

@@ -956,7 +956,8 @@ static bool launch_kw(const GemmParams &p, int kw, int nwg, hipStream_t st, cons
 }
 
 static void qgemm_check(const GemmParams &p) {
-    if (p.M < 1 || p.M > 128) throw BackendError("qgemm: M out of range");
+    // (32-bit buffer offsets: the inputs stay below 2 GiB)
+    if (p.M < 1 || p.M > 4096 || (int64_t)(p.M + 31) * p.K * 2 >= 0x80000000LL) throw BackendError("qgemm: M out of range");
     if (p.K % 256) throw BackendError("qgemm: K must be a multiple of 256");
     if (p.mode == GM_SWIGLU && (p.nseg != 2 || p.seg[0].rows != p.seg[1].rows || p.seg[0].fmt != p.seg[1].fmt))
         throw BackendError("qgemm: gate/up segments must match");

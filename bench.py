@@ -357,7 +357,7 @@ def main():
                             "step_algorithmic_bytes": int(tstep_bytes),
                             "k1_gbps": round(tb / tt / 1e9, 1),
                             "k1_frac": round(tb / tt / 1e9 / PEAK_HBM_GBPS, 4),
-                            "k1_kernel": "k_qgx (K1 for M>16)",
+                            "k1_kernel": "k_qwide (K1 for M>16)",
                             "k1_bytes_per_launch": int(tb / len(tg)),
                             "k1_avg_launch_us": round(tt / len(tg) * 1e6, 2),
                             "k1_traffic": measured_traffic("tree60")[0],
