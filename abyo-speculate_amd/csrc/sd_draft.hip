@@ -203,6 +203,14 @@ void launch_to_f16(const float *x, int64_t n, uint16_t *y, hipStream_t st) {
     hipLaunchKernelGGL(k_to_f16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, n, y);
 }
 
+__global__ void k_from_f16(const uint16_t *x, int64_t n, float *y) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) y[i] = h2f(x[i]);
+}
+void launch_from_f16(const uint16_t *x, int64_t n, float *y, hipStream_t st) {
+    hipLaunchKernelGGL(k_from_f16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, n, y);
+}
+
 // ---- RoPE, the draft cache append and attention, one wave per query head ----
 // q and this step's k rotated by the half-rotation RoPE at `pos` in f16
 // arithmetic (y1 = x1 c - x2 s, y2 = x1 s + x2 c, every product and sum

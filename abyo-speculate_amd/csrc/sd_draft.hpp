@@ -45,6 +45,7 @@ void launch_rmsnorm16(const DraftNorm &p, int rows, hipStream_t st);
 // out[0, H) = table[*id][0, H) (f16 rows; nothing written for an id out of range)
 void launch_gather16(const uint16_t *table, int64_t rows, int H, const int32_t *id, uint16_t *out, hipStream_t st);
 void launch_to_f16(const float *x, int64_t n, uint16_t *y, hipStream_t st);
+void launch_from_f16(const uint16_t *x, int64_t n, float *y, hipStream_t st);
 
 // RoPE of q and this step's k, the append of k and v to the draft cache, and
 // attention over every cached step, one launch
@@ -126,7 +127,9 @@ class Draft3 {
     // qkv [(nh + 2 nkv) hd], att [nh hd], after [H], xn [H], act [ffn], xf [H]
     uint16_t *x3 = nullptr, *hid[2] = {nullptr, nullptr}, *proj = nullptr, *comb = nullptr, *qkv = nullptr,
              *att = nullptr, *after = nullptr, *xn = nullptr, *act = nullptr, *xf = nullptr;
-    float *emb = nullptr, *logits = nullptr, *hin32 = nullptr;
+    float *emb = nullptr, *hin32 = nullptr;    // one block: input embedding [H] | hidden input [3H]
+    float *hid32 = nullptr, *logits = nullptr; // one block: step output [H] | logits
+    float *pin_io = nullptr;                   // pinned: step_host's inputs, then its outputs
     int32_t *tok = nullptr;                         // the current step's token id
     uint64_t *tk_part = nullptr;                    // top-k slice partials
     int *tk_cnt = nullptr;                          // top-k arrival count
@@ -193,6 +196,7 @@ class Draft2 {
     uint16_t *comb = nullptr, *xs = nullptr, *qkv = nullptr, *att = nullptr, *after = nullptr, *xn = nullptr,
              *act = nullptr, *xp = nullptr;
     float *hin32 = nullptr, *out32 = nullptr, *logits = nullptr;
+    float *pin_io = nullptr;  // pinned: step_host's inputs, then its output
     int32_t *tok = nullptr, *o_ids = nullptr, *o_dids = nullptr;  // o_ids | o_dids | o_lp: one block
     float *o_lp = nullptr;
     int32_t *pin = nullptr;  // pinned: the three output arrays, then the root token
