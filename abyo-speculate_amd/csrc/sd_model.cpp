@@ -160,7 +160,9 @@ void Model::alloc_buffers() {
     d_mask = (uint64_t *)(d_ids + 3 * Mx + (Mx & 1));
     d_src = dalloc<int>(Mx);
     d_prompt = dalloc<int>((size_t)2 * Rp);
-    qg_part_cap = std::max<int64_t>((int64_t)8 * Mx * std::max(qkvd, c.hidden), (int64_t)2 * Mx * 2 * c.ffn);
+    // K-slice partial sums: eight slices of a verify pass, up to four of a prompt chunk within 96 MB
+    qg_part_cap = std::max<int64_t>((int64_t)8 * Mx * std::max(qkvd, c.hidden),
+                                    std::min<int64_t>((int64_t)4 * Rp * std::max(qkvd, c.hidden), 24 << 20));
     qg_part = dalloc<float>((size_t)qg_part_cap);
     ssq = dalloc<float>((size_t)16 * (c.hidden / 16));
     acc_m = dalloc<float>(Mx);
@@ -1097,7 +1099,8 @@ void Decoder::advance(const uint32_t *tokens, size_t n, int logits_mode, bool wa
         int M, nw = 0;
         if (done < wide) {
             const size_t left = wide - done, chunks = (left + m.prompt_rows - 1) / m.prompt_rows;
-            M = (int)((left + chunks - 1) / chunks);
+            // even chunks, in whole 128-token blocks of the matmul
+            M = (int)std::min<size_t>({left, (size_t)m.prompt_rows, ((left + chunks - 1) / chunks + 127) / 128 * 128});
         } else {
             M = (int)std::min(mb, n - done);
         }

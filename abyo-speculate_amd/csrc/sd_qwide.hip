@@ -11,13 +11,15 @@
 // copy to LDS and every LDS read are contiguous and free of bank conflicts.
 //
 // What bounds it: per 32-row tile, token tile and superblock 16 MFMAs (17 ns
-// each on the card) against about 34 other vector instructions per two MFMA
-// steps (2 ns each), which issue beside another wave's MFMAs but not beside
-// their own wave's: instruction issue up to 64 rows, the MFMAs above.  Per
-// superblock and 128 rows 0.7 / 0.95 / 1.6 us at 1 / 2 / 4 token tiles, plus
-// 6 us per launch.  Gate/up of 2 x 14336 x 4096 Q4_K (weights in the caches)
-// at 27 / 60 / 128 rows: 18.3 / 23.3 / 35.7 us, where one 16-row tile per
-// wave with the activations in row order took 23.8 / 33.1 / 55.7 us.
+// each with the whole chip busy, when it clocks at 1.9 GHz) against about 17
+// other vector instructions per MFMA step (2 ns each), which issue beside
+// another wave's MFMAs but not beside their own wave's: instruction issue up to
+// 64 rows, the MFMAs above (1.28 us of 1.09 per superblock, 128 rows and 128
+// tokens on an idle chip).  A launch adds 6 us.  Gate/up of 2 x 14336 x 4096
+// Q4_K (weights in the caches) at 27 / 60 / 128 rows: 18.7 / 21.5 / 32.2 us,
+// where one 16-row tile per wave with the activations in row order took
+// 23.8 / 33.1 / 55.7 us; at 512 rows 148 us (812 TFLOP/s).
+//
 // Dequantisation to fp16: a code is OR'ed into the mantissa of 1024.0h
 // (0x6400 | q == 1024 + q) or, for a code already at bits 4-7, of 64.0h
 // (0x5400 | q << 4 == 64 + q); the offset is subtracted exactly and one packed
@@ -236,20 +238,21 @@ __device__ __forceinline__ void wide_body(const WideWave &W, floatx16 (&acc)[TT]
     uintx4 xs[2 * TT];
     typename F::D w[2];
     // superblocks past the last are read as the last and not multiplied
-    auto ldx = [&](int i) {
+    auto ldx = [&](int i, int k) {  // piece k of superblock i's activations
         const uint32_t so = (uint32_t)(min(i, n - 1) + W.sb0) * kXTile;
-#pragma unroll
-        for (int k = 0; k < 2 * TT; k++)
-            xs[k] = bld16(W.x, (uint32_t)tid * 16u, uni(W.xtile[k >> 1] + so + (uint32_t)(k & 1) * 8192u));
+        xs[k] = bld16(W.x, (uint32_t)tid * 16u, uni(W.xtile[k >> 1] + so + (uint32_t)(k & 1) * 8192u));
     };
     auto ldw = [&](typename F::D &d, int i) {
         F::load(d, W.w, W.wvo, uni((uint32_t)(min(i, n - 1) + W.sb0) * F::TBB), W.r, W.j, W.kh);
     };
-    auto put = [&](int i) {
-        uint8_t *to = lds + (i & 1) * STAGE + tid * 16;
-#pragma unroll
-        for (int k = 0; k < 2 * TT; k++) *(uintx4 *)(to + k * (kWideThreads * 16)) = xs[k];
+    auto put = [&](int i, int k) {
+        *(uintx4 *)(lds + (i & 1) * STAGE + tid * 16 + k * (kWideThreads * 16)) = xs[k];
     };
+    // Superblock i is multiplied; between its MFMA steps, a piece at a time, the
+    // activations of i + 1 go to the other LDS stage (every wave is past its
+    // reads of i - 1 there) and those of i + 2 are requested.  All at the
+    // step's start, the copies held the MFMAs up: ffn_down at 128 rows 95 us,
+    // 78 so.
     auto step = [&](const typename F::D &d, int i) {
         const uint8_t *xb = lds + (i & 1) * STAGE + W.kh * 8192 + lane * 16;
         typename F::S sc;
@@ -265,45 +268,41 @@ __device__ __forceinline__ void wide_body(const WideWave &W, floatx16 (&acc)[TT]
                 for (int tt = 0; tt < TT; tt++) b[(ks + 1) & 1][tt] = *(const half8 *)(xb + tt * kXTile + (ks + 1) * 1024);
                 a[(ks + 1) & 1] = F::frag(d, sc, (ks + 1) >> 1, (ks + 1) & 1);
             }
+            if (ks % (4 / TT) == 0) {
+                put(i + 1, ks / (4 / TT));
+                ldx(i + 2, ks / (4 / TT));
+            }
 #pragma unroll
             for (int tt = 0; tt < TT; tt++)
                 acc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks & 1], b[ks & 1][tt], acc[tt], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     // The loads' order is pinned: a wait on one load waits for every older one,
     // and the compiler's wait counts are exact only if the order before the
     // loop is the order inside it.
 #define PIN __builtin_amdgcn_sched_barrier(0)
-    ldx(0);
+#pragma unroll
+    for (int k = 0; k < 2 * TT; k++) ldx(0, k);
     PIN;
     ldw(w[0], 0);
     PIN;
-    put(0);
+#pragma unroll
+    for (int k = 0; k < 2 * TT; k++) put(0, k);
     PIN;
-    ldx(1);
+#pragma unroll
+    for (int k = 0; k < 2 * TT; k++) ldx(1, k);
     PIN;
     ldw(w[1], 1);
     PIN;
     __syncthreads();
-    // step i: the activations of superblock i + 1 go to the other LDS stage
-    // (every wave is past its reads of superblock i - 1 there), those of i + 2
-    // are requested, superblock i is multiplied, the weights of i + 2 are
-    // requested
     for (int i = 0;; i += 2) {
-        put(i + 1);
-        PIN;
-        ldx(i + 2);
-        PIN;
         step(w[0], i);
         PIN;
         if (i + 1 >= n) return;
         ldw(w[0], i + 2);
         PIN;
         __syncthreads();
-        put(i + 2);
-        PIN;
-        ldx(i + 3);
-        PIN;
         step(w[1], i + 1);
         PIN;
         if (i + 2 >= n) return;
@@ -514,13 +513,32 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WP
 static int wide_tt(int M) { return M <= 32 ? 1 : M <= 64 ? 2 : 4; }
 static int row_blocks(const GemmParams &p) { return (wide_groups(p) + kRG - 1) / kRG; }
 static int token_blocks(int M) { return (M + 32 * wide_tt(M) - 1) / (32 * wide_tt(M)); }
+// K slices, where the consumer of the output adds them.  Up to 64 rows as many
+// as bring the launch to 192 workgroups (the 60-node tree step at targets of
+// 96 / 128 / 192: 783 / 771 / 737 us).  Above, the count with the least time
+// by what a launch was measured to cost: rounds of 256 workgroups at 6 us plus
+// 1.9 us a superblock, and the partial sums written and read at 4 TB/s.  280
+// workgroups (3584 rows, 1251 tokens) take two rounds unsplit.
 int qwide_slices(const GemmParams &p) {
     if (!p.allow_split || (p.mode != GM_STORE && p.mode != GM_RESID)) return 1;
     const int wgs = row_blocks(p) * token_blocks(p.M), nsb = p.K / 256;
     const int64_t R = 16LL * p.ntiles;
-    int ks = 1;
-    while (ks < 8 && wgs * ks < 192 && 2 * ks <= nsb && (int64_t)2 * ks * p.M * R <= p.part_cap) ks *= 2;
-    return ks;
+    int best = 1;
+    double least = 0.0;
+    for (int ks = 1; ks <= 8 && ks <= nsb && (ks == 1 || ks * p.M * R <= p.part_cap); ks *= 2) {
+        if (p.M <= 64) {
+            best = ks;
+            if (wgs * ks >= 192) break;
+            continue;
+        }
+        const int rounds = (wgs * ks + 255) / 256;
+        const double us = rounds * (6.0 + 1.9 * nsb / ks) + (ks > 1 ? ks * p.M * R * 8.0 / 4e6 : 0.0);
+        if (ks == 1 || us < least) {
+            least = us;
+            best = ks;
+        }
+    }
+    return best;
 }
 int qwide_slots(const GemmParams &p) { return row_blocks(p) * (wide_tt(p.M) == 1 ? 2 : 1); }
 
