@@ -20,8 +20,8 @@
 // per tile, device-scope partials) or by a combine kernel, with the same
 // arithmetic; nothing to merge when one split covers all keys.  The same
 // workgroups also run inside the fused Q/K/V launch (sd_qgemm.hip).
-// keys_per_wave and the split boundaries depend on P only, so a query's result
-// does not depend on how many other queries share the call.
+// keys_per_wave and the split boundaries depend on P only there, so a query's
+// result does not depend on how many other queries share the call.
 #include <algorithm>
 #include <mutex>
 #include <vector>
@@ -196,9 +196,14 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2)
 // all its waves, so the cache leaves L2 once per query block.  Copies run
 // kTStages blocks ahead through registers (as many LDS stages, one barrier per
 // block).  Splits are a few blocks long, so the grid covers the chip; the
-// combine kernel merges them.  Sixteen waves of one tile each (four per SIMD)
-// hide the softmax's and the MFMAs' latencies better than eight of two.
-constexpr int kTWaves = 16;
+// combine kernel merges them.  Eight waves of one tile each: a block of keys
+// costs a workgroup half of what it costs sixteen (each wave reads all of it
+// from LDS), so the same CUs take half the splits in twice the blocks, and half
+// the partial rows are written and merged.  60 rows of 32 heads over 4096 keys,
+// with the merge: 37 us with sixteen waves and 26 splits, 23 with eight and 15
+// (four waves: 25; at 8192 keys 31, 28 and 32; at 1000 keys and 128 rows 22, 19
+// and 21).
+constexpr int kTWaves = 8;
 constexpr int kTThreads = 64 * kTWaves;
 constexpr int kTQW = 1;
 constexpr int kTStages = 3;
@@ -428,26 +433,25 @@ void launch_rope_kv(const RopeKvParams &p, hipStream_t st) {
     hipLaunchKernelGGL(k_rope_kv, dim3(p.M, (units + 63) / 64), dim3(64), 0, st, p);
 }
 
+// k_attn_t: splits of whole 32-key blocks, as many as the query blocks leave
+// CUs for (a workgroup fills a CU; one workgroup more than CUs is a second round:
+// 90 rows over 300 keys 15.2 against 19.6 us)
+AttnSplit attn_split_wide(int P, int M, int n_kv, int n_rep, int max_splits) {
+    const int T = P + M, nqt = (M * n_rep + 15) / 16, nqb = (nqt + kTWaves * kTQW - 1) / (kTWaves * kTQW);
+    const int want = std::max(1, std::min(max_splits, 256 / (n_kv * nqb)));
+    const int kps = ((T + want - 1) / want + 31) / 32 * 32;
+    return AttnSplit{kps / 4, (T + kps - 1) / kps};
+}
+
 // Up to 16 rows (a linear verify or a decode step) the key ranges are a
 // function of P alone, so each row's arithmetic is the same as in a one-row
 // call: a split is 8 waves x 3 steps of 32 keys below 1024 cached positions
 // (one split up to ~750), else 8 waves x as many steps as give about 64 / n_kv
 // splits; each wave's first two steps sit in its registers (requested while
-// the fused launch's matmul runs), later ones stream behind them.  Above 16
-// rows, the splits shrink as query blocks grow, towards one 8-wave workgroup
-// per CU (256).
+// the fused launch's matmul runs), later ones stream behind them.
 AttnSplit attn_split(int P, int M, int n_kv, int n_rep) {
     const int T = P + M;
-    if (M > 16) {
-        // k_attn_t: splits of kps keys (whole 32-key blocks), towards one
-        // workgroup per CU over the query blocks
-        const int nqt = (M * n_rep + 15) / 16, nqb = (nqt + kTWaves * kTQW - 1) / (kTWaves * kTQW);
-        int want = 256 / (n_kv * nqb);
-        want = want < 1 ? 1 : want > kTMaxSplits ? kTMaxSplits : want;
-        int kps = (P + 1 + want - 1) / want;
-        kps = kps < 32 ? 32 : (kps + 31) / 32 * 32;
-        return AttnSplit{kps / 4, (T + kps - 1) / kps};
-    }
+    if (M > 16) return attn_split_wide(P, M, n_kv, n_rep, kTMaxSplits);
     // steps per wave: 3 (one split) for short prefixes, else as few as give
     // about 64 / n_kv splits (64 workgroups per query tile), at most 32
     const int want = std::min(kTMaxSplits, n_kv >= 64 ? 1 : 64 / n_kv);
@@ -456,20 +460,9 @@ AttnSplit attn_split(int P, int M, int n_kv, int n_rep) {
     return AttnSplit{32 * spw, (T + kps - 1) / kps};
 }
 
-// k_attn_t over a prompt's rows: query blocks first, and where they leave CUs
-// idle, as many splits as fill them
-AttnSplit attn_split_causal(int P, int M, int n_kv, int n_rep, int max_splits) {
-    const int T = P + M, nqt = (M * n_rep + 15) / 16, nqb = (nqt + kTWaves * kTQW - 1) / (kTWaves * kTQW);
-    const int want = std::max(1, std::min(max_splits, 256 / (n_kv * nqb)));
-    const int kps = ((T + want - 1) / want + 31) / 32 * 32;
-    return AttnSplit{kps / 4, (T + kps - 1) / kps};
-}
-
-// above 16 rows the split size is >= (P + 1) / want and >= 32 with
-// want <= kTMaxSplits, so for M <= 128 nsplit = ceil((P + M) / size) <=
-// want + 1 + 128 / 32; up to 16 rows a split holds 768 keys below 1024
-// cached positions (nsplit <= 2) and >= (P + 1) / want above (nsplit <=
-// want + 1 <= kTMaxSplits + 1)
+// above 16 rows nsplit <= want <= kTMaxSplits; up to 16 rows a split holds 768
+// keys below 1024 cached positions (nsplit <= 2) and >= (P + 1) / want above
+// (nsplit <= want + 1 <= kTMaxSplits + 1)
 static_assert(kTMaxSplits + 5 <= kCombMaxSplits && kTMaxSplits + 5 <= kFusedMaxSplits, "split bounds");
 int attn_max_splits(int) { return kTMaxSplits + 5; }
 

@@ -27,17 +27,17 @@ struct RopeKvParams {
     float norm_eps;
 };
 
-// Work split of one attention call, a function of the prefix length P and the
-// head layout only (never of M), so a query's arithmetic does not depend on
-// how many other queries share the call.
+// Work split of one attention call: up to 16 rows a function of the prefix
+// length P and the head layout only (never of M), so a query's arithmetic does
+// not depend on how many other queries share the call.
 struct AttnSplit {
     int keys_per_wave;  // a split covers 4 * keys_per_wave keys (multiple of 32 up to 16 rows, of 8 above)
     int nsplit;         // workgroups along the keys (for T = P + M keys)
 };
 AttnSplit attn_split(int P, int M, int n_kv, int n_rep);
 int attn_max_splits(int n_kv);  // upper bound of nsplit over all P, M <= 128
-// the split of a prompt's M > 16 causal rows, at most max_splits
-AttnSplit attn_split_causal(int P, int M, int n_kv, int n_rep, int max_splits);
+// more than 16 rows (a prompt chunk's too), at most max_splits
+AttnSplit attn_split_wide(int P, int M, int n_kv, int n_rep, int max_splits);
 
 struct AttnParams {
     const uint16_t *q16;

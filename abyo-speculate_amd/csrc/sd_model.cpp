@@ -636,7 +636,7 @@ void Model::forward(const int *ids, const int *pos, const uint64_t *mask, int ma
     const int H = c.hidden, QD = c.q_dim(), KVD = c.kv_dim(), QKVD = QD + 2 * KVD;
     launch_embed(gw[K_TOK_EMBD].fmt, embed_table(), H, ids_dev, M, h, st);
     const int max_splits = (int)std::min<int64_t>(nsplit_max, part_rows / M);
-    const AttnSplit split = prompt ? attn_split_causal(P, M, c.n_kv_heads, c.n_heads / c.n_kv_heads, max_splits)
+    const AttnSplit split = prompt ? attn_split_wide(P, M, c.n_kv_heads, c.n_heads / c.n_kv_heads, max_splits)
                                    : attn_split(P, M, c.n_kv_heads, c.n_heads / c.n_kv_heads);
     if (split.nsplit > max_splits) throw BackendError("attention split count exceeds workspace");
     // M > 16 matmuls may leave K-slice partial sums in qg_part for the next

@@ -966,7 +966,7 @@ static void qgemm_check(const GemmParams &p) {
             if (p.seg[i].tile0 != p.seg[i - 1].tile0 + p.seg[i - 1].rows / 16)
                 throw BackendError("qgemm: segments must be consecutive");
     // fused RMSNorm and RoPE: both sides in the M <= 16 kernel's epilogues;
-    // above 16 rows (up to 64) only the input side, in k_qgx (its K slices
+    // above 16 rows (up to 64) only the input side, in k_qwide (its K slices
     // are scaled by the kernel that adds them)
     if ((p.next_w || p.rope.q16) && p.M > 16) throw BackendError("qgemm: fused output epilogues need M <= 16");
     if (p.norm_ssq && p.M <= 16 && p.norm_parts * 16 != p.K) throw BackendError("qgemm: norm partials must be one per 16 of K");
