@@ -237,8 +237,7 @@ sd_status sd_model_qmatmul_noalloc(sd_model *m, int32_t layer, int32_t kind, con
         setdev(m);
         // resolved at sd_model_create for this device; a kept pointer, no allocation
         void *scr = sd::noalloc_scratch(m->model->cfg.device);
-        m->model->qmatmul_into(layer, kind, x_dev, (int)rows, y_dev, (hipStream_t)stream, scr,
-                               sd::kNoAllocScratchBytes);
+        m->model->qmatmul_into(layer, kind, x_dev, (int)rows, y_dev, (hipStream_t)stream, scr);
     });
 }
 

@@ -197,12 +197,38 @@ __global__ __launch_bounds__(256) void k_norm_u(const float *x, const float *w, 
     }
 }
 
-// f32 rows -> fp16 fragment layout (hidden states handed to apply_lm_head)
-__global__ void k_to_frag16(const float *x, int K, uint16_t *out16, int ld16, int tiled) {
+// f32 rows -> a matmul's fp16 input; K % 4 == 0
+__global__ __launch_bounds__(256) void k_to_frag16(const float *x, int K, uint16_t *out16, int ld16, int tiled) {
     const int m = blockIdx.y;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = 4 * (blockIdx.x * 256 + threadIdx.x);
+    if (k >= K) return;
+    const float4 v = *(const float4 *)(x + (int64_t)m * K + k);
+    // elements k .. k+3 sit in fragment slots f, f+2, f+1, f+3: one 8-byte store
+    *(uint2 *)(out16 + act_index(m, k, ld16, tiled)) =
+        make_uint2((uint32_t)f2h(v.x) | ((uint32_t)f2h(v.z) << 16), (uint32_t)f2h(v.y) | ((uint32_t)f2h(v.w) << 16));
+}
+// the caller's rows may start anywhere a float may
+__global__ __launch_bounds__(256) void k_to_frag16_any(const float *x, int K, uint16_t *out16, int ld16, int tiled) {
+    const int m = blockIdx.y;
+    const int k = blockIdx.x * 256 + threadIdx.x;
     if (k >= K) return;
     out16[act_index(m, k, ld16, tiled)] = f2h(x[(int64_t)m * K + k]);
+}
+
+// y = the sum of nks slices of n floats, in slice order
+template <typename V> __global__ __launch_bounds__(256) void k_add_slices(const float *part, int nks, int64_t n, float *y) {
+    constexpr int W = sizeof(V) / 4;
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * W;
+    if (i >= n) return;
+    V a[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+        if (k < nks) a[k] = *(const V *)(part + k * n + i);
+    V s = a[0];
+#pragma unroll
+    for (int k = 1; k < 8; k++)
+        if (k < nks) s += a[k];
+    *(V *)(y + i) = s;
 }
 
 // ---- argmax over per-workgroup partials (first max wins, NaN/-inf skipped) ----
@@ -330,7 +356,16 @@ void launch_resid_u(float *x, const float *w, int M, int K, const float *part, i
     else hipLaunchKernelGGL(k_resid_u<64>, dim3(M, nb), dim3(64), 0, st, x, w, K, part, nks, ps, out16, ld16, ssq);
 }
 void launch_to_frag16(const float *x, int M, int K, uint16_t *out16, int ld16, hipStream_t st) {
-    hipLaunchKernelGGL(k_to_frag16, dim3((K + 255) / 256, M), dim3(256), 0, st, x, K, out16, ld16, M > 16 ? 1 : 0);
+    const int tiled = M > 16 ? 1 : 0;
+    if (K % 4 == 0 && (uintptr_t)x % 16 == 0)
+        hipLaunchKernelGGL(k_to_frag16, dim3((K + 1023) / 1024, M), dim3(256), 0, st, x, K, out16, ld16, tiled);
+    else hipLaunchKernelGGL(k_to_frag16_any, dim3((K + 255) / 256, M), dim3(256), 0, st, x, K, out16, ld16, tiled);
+}
+void launch_add_slices(const float *part, int nks, int64_t n, float *y, hipStream_t st) {
+    if (nks < 1 || nks > 8) throw BackendError("add_slices: 1 to 8 slices");
+    if (n % 4 == 0 && ((uintptr_t)part | (uintptr_t)y) % 16 == 0)
+        hipLaunchKernelGGL(k_add_slices<floatx4>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, st, part, nks, n, y);
+    else hipLaunchKernelGGL(k_add_slices<float>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, part, nks, n, y);
 }
 void launch_argmax_reduce(const float *pv, const int *pi, int nwg, int M, int *out, hipStream_t st) {
     hipLaunchKernelGGL(k_argmax_reduce, dim3(M), dim3(256), 0, st, pv, pi, nwg, out);

@@ -16,9 +16,12 @@ struct BackendError : std::runtime_error {
 // resolved with hipGetSymbolAddress on the first call for `device`, which must
 // be the current device; later calls return the kept address.
 // Calls stage at most kNoAllocMaxBytes of rows; above 16 rows they fill whole
-// tiles of 32 rows, less than twice as many.
+// tiles of 32 rows, less than twice as many.  K-slice partial sums of such
+// products follow the staged rows.
 constexpr size_t kNoAllocMaxBytes = (size_t)4 << 20;
-constexpr size_t kNoAllocScratchBytes = 2 * kNoAllocMaxBytes;
+constexpr size_t kNoAllocStageBytes = 2 * kNoAllocMaxBytes;
+constexpr size_t kNoAllocPartBytes = (size_t)24 << 20;
+constexpr size_t kNoAllocScratchBytes = kNoAllocStageBytes + kNoAllocPartBytes;
 void *noalloc_scratch(int device);
 
 // ---- sd_synth.hip ----

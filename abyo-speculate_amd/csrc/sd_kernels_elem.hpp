@@ -23,6 +23,8 @@ void launch_resid_u(float *x, const float *w, int M, int K, const float *part, i
                     float *ssq, hipStream_t st);
 // the fp16 rows of a matmul's input: operand order above 16 rows
 void launch_to_frag16(const float *x, int M, int K, uint16_t *out16, int ld16, hipStream_t st);
+// y[n] = the sum of nks <= 8 slices part[nks][n], in slice order
+void launch_add_slices(const float *part, int nks, int64_t n, float *y, hipStream_t st);
 // u = fp16(x * w) in fragment order + per-16-element sums of x^2 (ssq [M][K/16])
 // for a matmul with the RMSNorm fused into its epilogue
 void launch_norm_u(const float *x, const float *w, int M, int K, uint16_t *out16, int ld16, float *ssq,

@@ -464,46 +464,50 @@ void Model::qmatmul(int layer, int kind, const float *x, int M, float *y) {
     float *dx = dalloc<float>((size_t)M * t.K);
     float *dy = dalloc<float>((size_t)M * t.rows);
     uint16_t *dxp = dalloc<uint16_t>((size_t)(128 + 16) * t.K);
+    float *part = M > 16 ? dalloc<float>(kNoAllocPartBytes / 4) : nullptr;
     SD_HIP_CHECK(hipMemcpy(dx, x, (size_t)M * t.K * 4, hipMemcpyHostToDevice));
-    launch_to_frag16(dx, M, t.K, dxp, t.K, st);
-    GemmParams p{};
-    gemm_workspace(p);
-    p.seg[0] = seg_of(t, 0, dy, t.rows, 0, nullptr);
-    p.nseg = 1;
-    p.ntiles = t.rows / 16;
-    p.xp = dxp;
-    p.K = t.K;
-    p.M = M;
-    p.mode = GM_STORE;
-    launch_qgemm(p, st);
+    matmul_rows(t, dx, M, dy, dxp, part, st);
     SD_HIP_CHECK(hipStreamSynchronize(st));
     SD_HIP_CHECK(hipMemcpy(y, dy, (size_t)M * t.rows * 4, hipMemcpyDeviceToHost));
     hipFree(dx);
     hipFree(dy);
     hipFree(dxp);
+    if (part) hipFree(part);
+}
+
+// Above 16 rows K may be split (a 4096-row matrix alone is 32 workgroups): the
+// slices' sums go to `part` and are added in slice order.  14336 -> 4096
+// (Q6_K) at 40 rows 72 us unsplit, 17 + 4 so.
+void Model::matmul_rows(const DevTensor &t, const float *x, int M, float *y, uint16_t *staging, float *part,
+                        hipStream_t s) {
+    launch_to_frag16(x, M, t.K, staging, t.K, s);
+    GemmParams p{};
+    p.seg[0] = seg_of(t, 0, y, t.rows, 0, nullptr);
+    p.nseg = 1;
+    p.ntiles = t.rows / 16;
+    p.xp = staging;
+    p.K = t.K;
+    p.M = M;
+    p.mode = GM_STORE;
+    p.allow_split = M > 16;
+    p.part = part;
+    p.part_cap = kNoAllocPartBytes / 4;
+    launch_qgemm(p, s);
+    const int nks = qgemm_slices(p);
+    if (nks > 1) launch_add_slices(part, nks, (int64_t)M * t.rows, y, s);
 }
 
 void Model::qmatmul_into(int layer, int kind, const float *x_dev, int M, float *y_dev, hipStream_t stream,
-                         void *staging, size_t staging_bytes) {
+                         void *scratch) {
     DevTensor &t = slot(*this, layer, kind);
     if (!t.set() || t.fmt == F32) throw ArgError("qmatmul needs a quantised matrix tensor");
     if (M < 1 || M > 128) throw ArgError("rows must be in [1, 128]");
     if ((size_t)M * t.K * 2 > kNoAllocMaxBytes)
         throw ArgError("rows * K * 2 = " + std::to_string((size_t)M * t.K * 2) + " bytes of staged activations exceed the " +
                        std::to_string(kNoAllocMaxBytes) + "-byte scratch");
-    if ((size_t)(M > 16 ? (M + 31) / 32 * 32 : M) * t.K * 2 > staging_bytes)  // whole 32-row tiles
-        throw BackendError("staging too small");
-    hipStream_t s = stream ? stream : st;
-    launch_to_frag16(x_dev, M, t.K, (uint16_t *)staging, t.K, s);
-    GemmParams p{};  // allow_split = 0: no split-K partials
-    p.seg[0] = seg_of(t, 0, y_dev, t.rows, 0, nullptr);
-    p.nseg = 1;
-    p.ntiles = t.rows / 16;
-    p.xp = (const uint16_t *)staging;
-    p.K = t.K;
-    p.M = M;
-    p.mode = GM_STORE;
-    launch_qgemm(p, s);
+    static_assert(kNoAllocStageBytes >= 2 * kNoAllocMaxBytes, "whole 32-row tiles above 16 rows");
+    matmul_rows(t, x_dev, M, y_dev, (uint16_t *)scratch, (float *)((uint8_t *)scratch + kNoAllocStageBytes),
+                stream ? stream : st);
     SD_HIP_CHECK(hipGetLastError());
 }
 

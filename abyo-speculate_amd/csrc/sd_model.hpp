@@ -106,10 +106,9 @@ class Model {
     // raw matmul (test entry): y[M][N] = x[M][K] . W^T (x rounded to fp16)
     void qmatmul(int layer, int kind, const float *x, int M, float *y);
     // the same product on device buffers, enqueued on `stream` (the model's
-    // own stream when null), with the fp16 activations staged in `staging`
-    // (staging_bytes >= M * K * 2); allocates nothing and does not wait
-    void qmatmul_into(int layer, int kind, const float *x_dev, int M, float *y_dev, hipStream_t stream,
-                      void *staging, size_t staging_bytes);
+    // own stream when null), with the fp16 activations and K-slice sums in
+    // `scratch` (kNoAllocScratchBytes); allocates nothing and does not wait
+    void qmatmul_into(int layer, int kind, const float *x_dev, int M, float *y_dev, hipStream_t stream, void *scratch);
     // microbenchmark of one dequant-matmul launch: microseconds per launch
     enum { BENCH_QKV = 100, BENCH_GATE_UP = 101, BENCH_ALL_LAYERS = -2 };
     double bench_qmatmul(int layer, int kind, int M, int iters, double *bytes_out);
@@ -219,6 +218,9 @@ class Model {
 
   private:
     void alloc_buffers();
+    // y = x . W^T on `s`: staging holds the fp16 rows (whole 32-row tiles above
+    // 16), part kNoAllocPartBytes of K-slice sums
+    void matmul_rows(const DevTensor &t, const float *x, int M, float *y, uint16_t *staging, float *part, hipStream_t s);
     void run_gemm(GemmParams &p, int cls, double bytes);
     uint16_t *kc(int layer) const { return kv + (int64_t)layer * 2 * cfg.n_kv_heads * cap * cfg.head_dim; }
     uint16_t *vc(int layer) const { return kc(layer) + (int64_t)cfg.n_kv_heads * cap * cfg.head_dim; }

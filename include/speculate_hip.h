@@ -90,7 +90,7 @@ typedef struct sd_config {
     float rope_theta;     /* rope.freq_base */
     float rms_eps;        /* attention.layer_norm_rms_epsilon */
     int32_t ctx_len;      /* KV capacity in positions (context_length) */
-    int32_t max_batch;    /* rows of one forward pass (<= 128); longer observes are chunked */
+    int32_t max_batch;    /* rows of one verify pass (<= 128); observes beyond it take chunks of up to 2048 rows */
     int32_t tied_output;  /* 1: lm_head reuses token_embd (quantized_llama_local.rs:249-252) */
     int32_t device;       /* HIP device ordinal */
 } sd_config;
@@ -293,8 +293,9 @@ sd_status sd_synchronize(sd_model *m);
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  No counterpart in the reference.  x_dev [rows][K]
  * f32 and y_dev [rows][N] f32 are device buffers owned by the caller; the
- * fp16 activations are staged in a scratch array that every GPU the library
- * runs on holds once, 4 MiB (rows * K * 2 bytes must fit: SD_ERR_ARG beyond;
+ * fp16 activations and partial sums pass through a scratch array that every GPU
+ * the library runs on holds once (32 MiB, 4 MiB of them for the activations:
+ * rows * K * 2 bytes must fit, SD_ERR_ARG beyond;
  * rows <= 128).  The call enqueues on `stream` (a hipStream_t; NULL = the
  * handle's own stream) and returns without waiting.  All calls on one GPU
  * share its scratch: calls that overlap on one GPU (other streams, other

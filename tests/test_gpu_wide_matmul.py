@@ -2,12 +2,15 @@
 groups (128-row workgroups), one superblock of K, odd superblock counts and
 inputs one row past a tile, every format, against the kernel's own operands
 in f64 (fp16 activations times the emulated fp16 weights)."""
+import types
+
 import numpy as np
 import pytest
 
 import oracle as O
 from _models import MIX_IDS, hip_cfg, oracle_cfg, rel_err
 from test_gpu_kernels import operand_weights
+from test_zz_no_alloc import DevBuf, _hip_runtime, _noalloc
 
 pytestmark = pytest.mark.gpu
 
@@ -32,4 +35,31 @@ def test_tile_edges(hip, mix, M):
         ref = O.round_f16(x).astype(np.float64) @ operand_weights(fmt, raw, rows, K, M).astype(np.float64).T
         # f32 sums of K exact products: at most K ulps of the sum of magnitudes, far below in practice
         assert rel_err(y, ref) < K * 2.0 ** -24 * 8, (kind, rel_err(y, ref))
+    dec.close()
+
+
+def test_noalloc_split_unaligned_rows(hip):
+    """The allocation-free product with K slices (256 output rows, K = 7168: eight
+    slices) on inputs and outputs that start one float into an allocation."""
+    ocfg = oracle_cfg(mix="q4_k", n_layers=1, hidden=256, n_heads=4, n_kv_heads=1, head_dim=64, ffn=7168, vocab=256,
+                      ctx_len=64)
+    dec = hip.HipQuantDecoder(hip_cfg(hip, ocfg))
+    dec.synthesize(MIX_IDS["q4_k"], ocfg.seed, ocfg.weight_std)
+    rows, K = ocfg.shape(O.K_FFN_DOWN)
+    rt = _hip_runtime()
+    for M in (17, 40, 128):
+        x = np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)
+        exp = dec.qmatmul(0, O.K_FFN_DOWN, x)
+        for at in (0, 1):
+            xb, yb = DevBuf(rt, 4 * (M * K + 4)), DevBuf(rt, 4 * (M * rows + 4))
+            xb.put(np.concatenate([np.zeros(at, np.float32), x.reshape(-1)]))
+            yb.put(np.zeros(M * rows + 4, np.float32))
+            xo, yo = types.SimpleNamespace(p=xb.p.value + 4 * at), types.SimpleNamespace(p=yb.p.value + 4 * at)
+            assert _noalloc(hip, dec, 0, O.K_FFN_DOWN, xo, M, yo) == 0
+            dec.synchronize()
+            got = yb.get(M * rows + 4)
+            assert np.array_equal(got[at:at + M * rows].view(np.uint32), exp.reshape(-1).view(np.uint32)), (M, at)
+            assert not got[at + M * rows:].any()
+            xb.free()
+            yb.free()
     dec.close()
