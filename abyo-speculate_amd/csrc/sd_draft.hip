@@ -218,8 +218,14 @@ void launch_from_f16(const uint16_t *x, int64_t n, float *y, hipStream_t st) {
 // one, softmax in f32 rounded to f16, out = f16(sum_j p_j v_j).  Every wave of
 // a kv head rotates that head's k itself; the first of them appends k and v to
 // slot `step` of the caches, which later steps read.  A lane holds the
-// rotation pairs (i, i + hd/2) for i = lane and lane + 64.
+// rotation pairs (i, i + hd/2) for i = lane and lane + 64.  One wave's chain of
+// loads and cross-lane sums bounds it, so the kernel is compiled for NS steps
+// and NP pairs and the launch takes the least that hold the call's (steps past
+// T add nothing): 10.0 us a launch
+// as one kernel for 16 steps and two pairs, a draft step (with the top-k below)
+// 12 us less.  The values are requested with the keys, not after the scores.
 constexpr int kAttnPairs = 2;  // head_dim up to 256
+template <int NS, int NP>
 __global__ __launch_bounds__(64) void k_draft_attn(DraftAttn p) {
     warm_kernargs<sizeof(DraftAttn)>();
     const int h = blockIdx.x, lane = threadIdx.x;
@@ -229,10 +235,10 @@ __global__ __launch_bounds__(64) void k_draft_attn(DraftAttn p) {
     const uint16_t *qg = p.qkv + (int64_t)h * hd;
     const uint16_t *kg = p.qkv + (int64_t)(p.n_heads + kv) * hd;
     const uint16_t *vg = p.qkv + (int64_t)(p.n_heads + p.n_kv + kv) * hd;
-    _Float16 q1[kAttnPairs], q2[kAttnPairs], k1[kAttnPairs], k2[kAttnPairs];
-    float v1[kAttnPairs], v2[kAttnPairs];
+    _Float16 q1[NP], q2[NP], k1[NP], k2[NP];
+    float v1[NP], v2[NP];
 #pragma unroll
-    for (int e = 0; e < kAttnPairs; e++) {
+    for (int e = 0; e < NP; e++) {
         const int i = lane + 64 * e;
         const int ic = i < half ? i : 0;
         const _Float16 c = __builtin_bit_cast(_Float16, cs[ic]), sv = __builtin_bit_cast(_Float16, sn[ic]);
@@ -252,7 +258,7 @@ __global__ __launch_bounds__(64) void k_draft_attn(DraftAttn p) {
         uint16_t *kd = p.kcache + ((int64_t)p.step * p.n_kv + kv) * hd;
         uint16_t *vd = p.vcache + ((int64_t)p.step * p.n_kv + kv) * hd;
 #pragma unroll
-        for (int e = 0; e < kAttnPairs; e++) {
+        for (int e = 0; e < NP; e++) {
             const int i = lane + 64 * e;
             if (i < half) {
                 kd[i] = __builtin_bit_cast(uint16_t, k1[e]);
@@ -262,16 +268,28 @@ __global__ __launch_bounds__(64) void k_draft_attn(DraftAttn p) {
             }
         }
     }
-    // scores: the cached steps' keys loaded in one batch (clamped to slot 0
-    // past the cached ones, every load issued), this step's from registers
-    float sc[kDraftMaxSteps];
+    // scores: the cached steps' keys and values loaded in one batch (clamped to
+    // slot 0 past the cached ones, every load issued), this step's from registers
+    uint16_t vr1[NS][NP], vr2[NS][NP];
 #pragma unroll
-    for (int j = 0; j < kDraftMaxSteps; j++) {
+    for (int j = 0; j < NS; j++) {
+        const uint16_t *vj = p.vcache + ((int64_t)(j < T - 1 ? j : 0) * p.n_kv + kv) * hd;
+#pragma unroll
+        for (int e = 0; e < NP; e++) {
+            const int i = lane + 64 * e;
+            const int ic = i < half ? i : 0;
+            vr1[j][e] = vj[ic];
+            vr2[j][e] = vj[ic + half];
+        }
+    }
+    float sc[NS];
+#pragma unroll
+    for (int j = 0; j < NS; j++) {
         const int jc = j < T - 1 ? j : 0;
         const uint16_t *kj = p.kcache + ((int64_t)jc * p.n_kv + kv) * hd;
         float a = 0.f, b = 0.f;
 #pragma unroll
-        for (int e = 0; e < kAttnPairs; e++) {
+        for (int e = 0; e < NP; e++) {
             const int i = lane + 64 * e;
             const int ic = i < half ? i : 0;
             const float c1 = h2f(kj[ic]), c2 = h2f(kj[ic + half]);
@@ -284,7 +302,7 @@ __global__ __launch_bounds__(64) void k_draft_attn(DraftAttn p) {
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < kDraftMaxSteps; j++) {
+    for (int j = 0; j < NS; j++) {
         float a = sc[j];
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o);
@@ -293,21 +311,17 @@ __global__ __launch_bounds__(64) void k_draft_attn(DraftAttn p) {
     }
     float sum = 0.f;
 #pragma unroll
-    for (int j = 0; j < kDraftMaxSteps; j++) {
+    for (int j = 0; j < NS; j++) {
         sc[j] = j < T ? expf(sc[j] - mx) : 0.f;
         sum += sc[j];
     }
-    float o1[kAttnPairs] = {}, o2[kAttnPairs] = {};
+    float o1[NP] = {}, o2[NP] = {};
 #pragma unroll
-    for (int j = 0; j < kDraftMaxSteps; j++) {
+    for (int j = 0; j < NS; j++) {
         const float pj = r16(sc[j] / sum);
-        const int jc = j < T - 1 ? j : 0;
-        const uint16_t *vj = p.vcache + ((int64_t)jc * p.n_kv + kv) * hd;
 #pragma unroll
-        for (int e = 0; e < kAttnPairs; e++) {
-            const int i = lane + 64 * e;
-            const int ic = i < half ? i : 0;
-            const float c1 = h2f(vj[ic]), c2 = h2f(vj[ic + half]);
+        for (int e = 0; e < NP; e++) {
+            const float c1 = h2f(vr1[j][e]), c2 = h2f(vr2[j][e]);
             const float a = j < T - 1 ? c1 : v1[e], b = j < T - 1 ? c2 : v2[e];
             if (j < T) {
                 o1[e] += pj * a;
@@ -316,7 +330,7 @@ __global__ __launch_bounds__(64) void k_draft_attn(DraftAttn p) {
         }
     }
 #pragma unroll
-    for (int e = 0; e < kAttnPairs; e++) {
+    for (int e = 0; e < NP; e++) {
         const int i = lane + 64 * e;
         if (i < half) {
             p.out[(int64_t)h * hd + i] = f2h(o1[e]);
@@ -327,7 +341,12 @@ __global__ __launch_bounds__(64) void k_draft_attn(DraftAttn p) {
 void launch_draft_attn(const DraftAttn &p, hipStream_t st) {
     if (p.step < 0 || p.step >= kDraftMaxSteps) throw BackendError("draft attention: steps out of range");
     if (p.hd % 2 || p.hd > 128 * kAttnPairs || p.n_heads % p.n_kv) throw BackendError("draft attention: head layout");
-    hipLaunchKernelGGL(k_draft_attn, dim3(p.n_heads), dim3(64), 0, st, p);
+    const int T = p.step + 1;
+    const dim3 g(p.n_heads), b(64);
+    if (p.hd > 128) hipLaunchKernelGGL((k_draft_attn<kDraftMaxSteps, kAttnPairs>), g, b, 0, st, p);
+    else if (T <= 4) hipLaunchKernelGGL((k_draft_attn<4, 1>), g, b, 0, st, p);
+    else if (T <= 8) hipLaunchKernelGGL((k_draft_attn<8, 1>), g, b, 0, st, p);
+    else hipLaunchKernelGGL((k_draft_attn<kDraftMaxSteps, 1>), g, b, 0, st, p);
 }
 
 // ---- top-k, log-probs and the next step's token --------------------------------
@@ -336,43 +355,59 @@ void launch_draft_attn(const DraftAttn &p, hipStream_t st) {
 // -inf, and its top k by (value descending, index ascending)
 // (medusa.rs:477-487; NaN after every number, NaNs by index), found in k
 // selection rounds (each takes the first item of the order after the previous
-// winner).  The last workgroup to finish merges the slices in slice order:
-// M = max m, S = sum over slices of s exp(m - M) (NaN when every logit is
-// -inf, as the reference's sum of exp(-inf - -inf) is), lse = ln S + M, and
-// the top k of the slices' candidates.  Outputs the draft ids, l_i - lse, the
+// winner).  The last workgroup to finish merges the slices:
+// M = max m, S = sum over slices of s exp(m - M) (64 lanes' sums, added in a
+// fixed order; NaN when every logit is -inf, as the reference's sum of
+// exp(-inf - -inf) is), lse = ln S + M, and the top k of the slices' candidates.
+// A (value, index) pair is one 64-bit key whose unsigned order is the selection
+// order, so a round is a maximum over keys: across lanes in four DPP and two
+// permlane-swap steps, where pairs compared field by field through LDS shuffles
+// and the slices' sums added one after the other took 14.5 us at
+// 32 slices.  Outputs the draft ids, l_i - lse, the
 // target ids through d2t, and the top-1 target id as the next step's token.
 constexpr int kTkT = 256, kTkPer = 4, kTkSlice = kTkT * kTkPer, kTkMaxSlices = 256, kTkLaneSlices = kTkMaxSlices / 64;
 static_assert(kTkSlice * kTkMaxSlices >= 262144, "draft top-k slices");
-__device__ __forceinline__ bool tk_before(float v1, int i1, float v2, int i2) {
-    const bool n1 = v1 != v1, n2 = v2 != v2;
-    if (n1 || n2) return n1 == n2 ? i1 < i2 : n2;
-    return v1 > v2 || (v1 == v2 && i1 < i2);
+// larger is first: value descending (-0 as +0, NaN after every number), then
+// index ascending.  0 is no key.
+__device__ __forceinline__ uint64_t tk_key(float v, int i) {
+    const uint32_t u = __float_as_uint(v == 0.f ? 0.f : v);
+    const uint32_t o = v != v ? 0u : u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
+    return (uint64_t)o << 32 | (uint32_t)~i;
 }
-__device__ __forceinline__ void tk_wave_best(float &bv, int &bi) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(bv, o);
-        const int oi = __shfl_xor(bi, o);
-        if (tk_before(ov, oi, bv, bi)) {
-            bv = ov;
-            bi = oi;
-        }
-    }
+__device__ __forceinline__ float tk_value(uint64_t k) {
+    const uint32_t o = (uint32_t)(k >> 32);
+    return o == 0 ? NAN : __uint_as_float(o >> 31 ? o ^ 0x80000000u : ~o);
 }
-__device__ __forceinline__ void tk_st64(uint64_t *p, float a, uint32_t b) {
-    __hip_atomic_store(p, (uint64_t)__float_as_uint(a) | ((uint64_t)b << 32), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ int tk_index(uint64_t k) { return (int)~(uint32_t)k; }
+__device__ __forceinline__ uint64_t tk_max(uint64_t a, uint64_t b) { return a > b ? a : b; }
+template <int CTRL> __device__ __forceinline__ uint64_t tk_dpp_max(uint64_t k) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)k, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(k >> 32), CTRL, 0xf, 0xf, true);
+    return tk_max(k, (uint64_t)hi << 32 | lo);
 }
-__device__ __forceinline__ void tk_ld64(const uint64_t *p, float &a, int &b) {
-    const uint64_t u = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    a = __uint_as_float((uint32_t)u);
-    b = (int)(uint32_t)(u >> 32);
+// the wave's largest key, on every lane (the whole wave takes part)
+__device__ __forceinline__ uint64_t tk_wave_max(uint64_t k) {
+    k = tk_dpp_max<0xB1>(k);   // lane ^ 1
+    k = tk_dpp_max<0x4E>(k);   // lane ^ 2
+    k = tk_dpp_max<0x141>(k);  // mirrored in 8: the other four lanes
+    k = tk_dpp_max<0x140>(k);  // mirrored in 16: the other eight
+    const auto l16 = __builtin_amdgcn_permlane16_swap((uint32_t)k, (uint32_t)k, false, false);
+    const auto h16 = __builtin_amdgcn_permlane16_swap((uint32_t)(k >> 32), (uint32_t)(k >> 32), false, false);
+    k = tk_max((uint64_t)h16[0] << 32 | l16[0], (uint64_t)h16[1] << 32 | l16[1]);
+    const auto l32 = __builtin_amdgcn_permlane32_swap((uint32_t)k, (uint32_t)k, false, false);
+    const auto h32 = __builtin_amdgcn_permlane32_swap((uint32_t)(k >> 32), (uint32_t)(k >> 32), false, false);
+    return tk_max((uint64_t)h32[0] << 32 | l32[0], (uint64_t)h32[1] << 32 | l32[1]);
 }
-constexpr int kTkNone = 0x7fffffff;
+__device__ __forceinline__ void tk_st64(uint64_t *p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t tk_ld64(const uint64_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __global__ __launch_bounds__(kTkT) void k_draft_topk(DraftTopk p) {
     warm_kernargs<sizeof(DraftTopk)>();
-    __shared__ float sv[2][kTkT / 64], red[kTkT / 64], wv[kDraftMaxTopk];
-    __shared__ int si[2][kTkT / 64], wi[kDraftMaxTopk];
+    __shared__ float red[kTkT / 64];
+    __shared__ uint64_t sk[2][kTkT / 64], wk[kDraftMaxTopk];
     __shared__ int s_last;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, sl = blockIdx.x, nsl = gridDim.x;
     float v[kTkPer];
@@ -399,44 +434,27 @@ __global__ __launch_bounds__(kTkT) void k_draft_topk(DraftTopk p) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
     if (lane == 0) red[wave] = s;
-    float lv = 0.f;
-    int li = -1;
+    uint64_t key[kTkPer], last_k = ~0ull;
+#pragma unroll
+    for (int j = 0; j < kTkPer; j++) key[j] = xi[j] < p.V ? tk_key(v[j], xi[j]) : 0;
     for (int r = 0; r < p.k; r++) {
-        float bv = NAN;
-        int bi = kTkNone;
+        uint64_t best = 0;
 #pragma unroll
-        for (int j = 0; j < kTkPer; j++) {
-            const bool elig = xi[j] < p.V && (li < 0 || tk_before(lv, li, v[j], xi[j]));
-            if (elig && tk_before(v[j], xi[j], bv, bi)) {
-                bv = v[j];
-                bi = xi[j];
-            }
-        }
-        tk_wave_best(bv, bi);
-        if (lane == 0) {
-            sv[r & 1][wave] = bv;
-            si[r & 1][wave] = bi;
-        }
+        for (int j = 0; j < kTkPer; j++) best = tk_max(best, key[j] < last_k ? key[j] : 0);
+        best = tk_wave_max(best);
+        if (lane == 0) sk[r & 1][wave] = best;
         __syncthreads();
-        bv = sv[r & 1][0];
-        bi = si[r & 1][0];
+        best = sk[r & 1][0];
 #pragma unroll
-        for (int w = 1; w < kTkT / 64; w++)
-            if (tk_before(sv[r & 1][w], si[r & 1][w], bv, bi)) {
-                bv = sv[r & 1][w];
-                bi = si[r & 1][w];
-            }
-        lv = bv;
-        li = bi;
-        if (t == 0) {
-            wv[r] = bv;
-            wi[r] = bi;
-        }
+        for (int w = 1; w < kTkT / 64; w++) best = tk_max(best, sk[r & 1][w]);
+        last_k = best;
+        if (t == 0) wk[r] = best;
     }
     if (t == 0) {
         uint64_t *pp = p.part + (int64_t)sl * (1 + kDraftMaxTopk);
-        tk_st64(pp, mx, __float_as_uint((red[0] + red[1]) + (red[2] + red[3])));
-        for (int r = 0; r < p.k; r++) tk_st64(pp + 1 + r, wv[r], (uint32_t)wi[r]);
+        tk_st64(pp, (uint64_t)__float_as_uint(mx) |
+                        (uint64_t)__float_as_uint((red[0] + red[1]) + (red[2] + red[3])) << 32);
+        for (int r = 0; r < p.k; r++) tk_st64(pp + 1 + r, wk[r]);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partials are stored before the count
         const int last = __hip_atomic_fetch_add(p.cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsl - 1;
         if (last) __hip_atomic_store(p.cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -445,67 +463,53 @@ __global__ __launch_bounds__(kTkT) void k_draft_topk(DraftTopk p) {
     __syncthreads();
     if (!s_last || wave != 0) return;
     // the merge, one wave: lane l holds slices l, l + 64, ... (kTkLaneSlices of them)
-    float cv[kTkLaneSlices * kDraftMaxTopk];
-    int ci[kTkLaneSlices * kDraftMaxTopk];
+    uint64_t ck[kTkLaneSlices][kDraftMaxTopk];
     float m_l[kTkLaneSlices], s_l[kTkLaneSlices];
 #pragma unroll
     for (int q = 0; q < kTkLaneSlices; q++) {
         const int w = lane + 64 * q;
         m_l[q] = -INFINITY;
         s_l[q] = 0.f;
+        const uint64_t *pp = p.part + (int64_t)w * (1 + kDraftMaxTopk);
         if (w < nsl) {
-            int sb;
-            tk_ld64(p.part + (int64_t)w * (1 + kDraftMaxTopk), m_l[q], sb);
-            s_l[q] = __int_as_float(sb);
+            const uint64_t u = tk_ld64(pp);
+            m_l[q] = __uint_as_float((uint32_t)u);
+            s_l[q] = __uint_as_float((uint32_t)(u >> 32));
         }
 #pragma unroll
-        for (int r = 0; r < kDraftMaxTopk; r++) {
-            float a = NAN;
-            int b = kTkNone;
-            if (w < nsl && r < p.k) tk_ld64(p.part + (int64_t)w * (1 + kDraftMaxTopk) + 1 + r, a, b);
-            cv[q * kDraftMaxTopk + r] = a;
-            ci[q * kDraftMaxTopk + r] = (b < 0 || b >= p.V) ? kTkNone : b;
-        }
+        for (int r = 0; r < kDraftMaxTopk; r++) ck[q][r] = w < nsl && r < p.k ? tk_ld64(pp + 1 + r) : 0;
     }
     float M = -INFINITY;
 #pragma unroll
     for (int q = 0; q < kTkLaneSlices; q++) M = fmaxf(M, m_l[q]);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
-    float S = 0.f;  // in slice order, the same on every lane
-    for (int w = 0; w < nsl; w++) {
-        float mw = 0.f, sw = 0.f;
+    float S = 0.f;
 #pragma unroll
-        for (int q = 0; q < kTkLaneSlices; q++)
-            if (w >> 6 == q) {
-                mw = __shfl(m_l[q], w & 63);
-                sw = __shfl(s_l[q], w & 63);
-            }
-        if (mw != -INFINITY) S += sw * expf(mw - M);
-    }
+    for (int q = 0; q < kTkLaneSlices; q++)
+        if (m_l[q] != -INFINITY) S += s_l[q] * expf(m_l[q] - M);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) S += __shfl_xor(S, o);
     if (M == -INFINITY) S = NAN;
     const float lse = logf(S) + M;
-    float lv2 = 0.f;
-    int li2 = -1;
+    last_k = ~0ull;
     for (int r = 0; r < p.k; r++) {
-        float bv = NAN;
-        int bi = kTkNone;
+        uint64_t best = 0;
 #pragma unroll
-        for (int j = 0; j < kTkLaneSlices * kDraftMaxTopk; j++) {
-            const bool elig = ci[j] != kTkNone && (li2 < 0 || tk_before(lv2, li2, cv[j], ci[j]));
-            if (elig && tk_before(cv[j], ci[j], bv, bi)) {
-                bv = cv[j];
-                bi = ci[j];
-            }
+        for (int q = 0; q < kTkLaneSlices; q++) {
+            if (64 * q >= nsl) break;  // uniform
+#pragma unroll
+            for (int c = 0; c < kDraftMaxTopk; c++)
+                if (c < p.k) best = tk_max(best, ck[q][c] < last_k ? ck[q][c] : 0);
         }
-        tk_wave_best(bv, bi);
-        lv2 = bv;
-        li2 = bi;
+        best = tk_wave_max(best);
+        last_k = best;
         if (lane == 0) {
-            const bool ok = bi >= 0 && bi < p.V;
+            const int bi = tk_index(best);
+            const bool ok = best != 0 && bi >= 0 && bi < p.V;
             const int tgt = ok ? (p.d2t ? p.d2t[bi] : bi) : -1;
             p.out_draft[r] = ok ? bi : -1;
-            p.out_lp[r] = ok ? bv - lse : NAN;
+            p.out_lp[r] = ok ? tk_value(best) - lse : NAN;
             p.out_target[r] = tgt;
             if (r == 0) *p.next_token = ok ? tgt : 0;
         }

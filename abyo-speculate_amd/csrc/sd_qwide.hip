@@ -14,8 +14,8 @@
 // each with the whole chip busy, when it clocks at 1.9 GHz) against about 17
 // other vector instructions per MFMA step (2 ns each), which issue beside
 // another wave's MFMAs but not beside their own wave's: instruction issue up to
-// 64 rows, the MFMAs above (1.28 us of 1.09 per superblock, 128 rows and 128
-// tokens on an idle chip).  A launch adds 6 us.  Gate/up of 2 x 14336 x 4096
+// 64 rows, the MFMAs above (a superblock of 128 rows and 128 tokens takes 1.28 us, its
+// MFMAs 1.09).  A launch adds 6 us.  Gate/up of 2 x 14336 x 4096
 // Q4_K (weights in the caches) at 27 / 60 / 128 rows: 18.7 / 21.5 / 32.2 us,
 // where one 16-row tile per wave with the activations in row order took
 // 23.8 / 33.1 / 55.7 us; at 512 rows 148 us (812 TFLOP/s).

@@ -124,6 +124,23 @@ def test_draft_cache_limit(hip):
     d.close()
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(16, 4), (4, 2), (2, 1)])
+def test_attention_at_every_step(hip, heads, kv_heads):
+    """Each number of cached steps, 0 to 15, at head sizes 32, 128 and 256: the
+    attention is compiled for 4, 8 and 16 steps and for heads up to 128 and 256.
+    Both sides take the same inputs at each step, so TOL is the one step's
+    tolerance of the chain test above."""
+    d, c = _draft(hip, n_heads=heads, n_kv_heads=kv_heads)
+    o, _ = _oracle_of(hip, d, c)
+    rng = np.random.default_rng(heads)
+    for s in range(hip.DRAFT3_MAX_STEPS):
+        x, emb = rng.standard_normal((2, c["hidden"])).astype(np.float32)
+        out_d, _ = d.forward_hidden(x, emb, 3 + s)
+        out_o = o.forward_hidden(x, emb, 3 + s)
+        assert rel_err(out_d, out_o) < TOL, (heads, s, rel_err(out_d, out_o))
+    d.close()
+
+
 def _target(hip, prefix_len=40, seed=3):
     ocfg = oracle_cfg()
     om = O.OracleModel(ocfg)
@@ -305,6 +322,21 @@ def test_round_top_k_ties_across_slices(hip):
         lse = np.log(3 * np.exp(a) + 3 * np.exp(-a) + (V - 6))
         assert np.allclose(lps[s], [a - lse] * 3 + [-lse] * 5, atol=1e-5)
         assert ids[s] == [int(d2t[i]) for i in dids[s]]
+    d.close()
+    hd.close()
+
+
+def test_round_top_k_orders_nan_last(hip):
+    """NaN logits rank after every number, and among themselves by index."""
+    od, hd, prefix = _target(hip, prefix_len=12)
+    d, c = _draft(hip)
+    lm = np.full((c["draft_vocab"], c["hidden"]), np.nan, np.float16)
+    u = (np.random.default_rng(4).standard_normal(c["hidden"]) * 0.05).astype(np.float16)
+    lm[3100], lm[40], lm[2050] = u, 0, -u
+    d.set_tensor(hip.D3_LM_HEAD, lm)
+    ids, lps, dids = d.round(hd, [0, 1, 2], 1, 8)
+    assert dids[0] in ([3100, 40, 2050, 0, 1, 2, 3, 4], [2050, 40, 3100, 0, 1, 2, 3, 4])
+    assert np.isnan(lps[0]).all()
     d.close()
     hd.close()
 
