@@ -253,19 +253,48 @@ void Draft3::step_device(int position, bool first, hipStream_t st, int k, int32_
         g.y16 = in_h;
         launch_gemv16(DG_STORE, g, st);
     }
-    DraftNorm n{};
-    n.x32[0] = emb;
-    n.w[0] = w + off[D3_IN_NORM];
-    n.out[0] = comb;
-    n.x16[1] = in_h;
-    n.w[1] = w + off[D3_HID_NORM];
-    n.out[1] = comb + H;
-    n.H = H;
-    n.eps = c.rms_eps;
-    launch_rmsnorm16(n, 2, st);
+    const bool fuse = gemv16_norm_fits(H);
+    // the product's x: RMSNorm of `in` by the tensor wk, in its launch if the row fits
+    auto normed = [&](DraftGemv &g, const uint16_t *in, int wk, uint16_t *tmp) {
+        g.x = fuse ? in : tmp;
+        if (fuse) {
+            g.norm = 1;
+            g.H = H;
+            g.eps = c.rms_eps;
+            g.nw[0] = w + off[wk];
+            return;
+        }
+        DraftNorm n{};
+        n.x16[0] = in;
+        n.w[0] = w + off[wk];
+        n.out[0] = tmp;
+        n.H = H;
+        n.eps = c.rms_eps;
+        launch_rmsnorm16(n, 1, st);
+    };
     DraftGemv g{};
+    if (fuse) {
+        g.norm = 2;
+        g.H = H;
+        g.eps = c.rms_eps;
+        g.nx32 = emb;
+        g.nw[0] = w + off[D3_IN_NORM];
+        g.x = in_h;
+        g.nw[1] = w + off[D3_HID_NORM];
+    } else {
+        DraftNorm n{};
+        n.x32[0] = emb;
+        n.w[0] = w + off[D3_IN_NORM];
+        n.out[0] = comb;
+        n.x16[1] = in_h;
+        n.w[1] = w + off[D3_HID_NORM];
+        n.out[1] = comb + H;
+        n.H = H;
+        n.eps = c.rms_eps;
+        launch_rmsnorm16(n, 2, st);
+        g.x = comb;
+    }
     g.w = w + off[D3_Q];  // Q, K, V adjacent: one [(nh + 2 nkv) hd][2H] product
-    g.x = comb;
     g.N = (nh + 2 * nkv) * hd;
     g.K = 2 * H;
     g.y16 = qkv;
@@ -292,16 +321,9 @@ void Draft3::step_device(int position, bool first, hipStream_t st, int k, int32_
     g.y16 = after;
     g.res16 = in_h;  // attn_out + projected_features
     launch_gemv16(DG_ADD, g, st);
-    DraftNorm n1{};
-    n1.x16[0] = after;
-    n1.w[0] = w + off[D3_POST_NORM];
-    n1.out[0] = xn;
-    n1.H = H;
-    n1.eps = c.rms_eps;
-    launch_rmsnorm16(n1, 1, st);
     g = DraftGemv{};
     g.w = w + off[D3_GATE];  // GATE, UP adjacent
-    g.x = xn;
+    normed(g, after, D3_POST_NORM, xn);
     g.N = c.ffn;
     g.K = H;
     g.y16 = act;
@@ -314,16 +336,9 @@ void Draft3::step_device(int position, bool first, hipStream_t st, int k, int32_
     g.y16 = out_h;
     g.res16 = after;
     launch_gemv16(DG_ADD, g, st);
-    DraftNorm n2{};
-    n2.x16[0] = out_h;
-    n2.w[0] = w + off[D3_NORM];
-    n2.out[0] = xf;
-    n2.H = H;
-    n2.eps = c.rms_eps;
-    launch_rmsnorm16(n2, 1, st);
     g = DraftGemv{};
     g.w = w + off[D3_LM_HEAD];
-    g.x = xf;
+    normed(g, out_h, D3_NORM, xf);
     g.N = c.draft_vocab;
     g.K = H;
     g.y32 = logits;
@@ -572,16 +587,24 @@ void Draft2::step_device(int position, hipStream_t st) {
     g.y16 = after;
     g.res16 = xs;  // attn + res
     launch_gemv16(DG_ADD, g, st);
-    DraftNorm n{};
-    n.x16[0] = after;
-    n.w[0] = w + off[D2_POST_NORM];
-    n.out[0] = xn;
-    n.H = H;
-    n.eps = c.rms_eps;
-    launch_rmsnorm16(n, 1, st);
     g = DraftGemv{};
     g.w = w + off[D2_GATE];  // GATE, UP adjacent
-    g.x = xn;
+    if (gemv16_norm_fits(H)) {
+        g.x = after;
+        g.norm = 1;
+        g.H = H;
+        g.eps = c.rms_eps;
+        g.nw[0] = w + off[D2_POST_NORM];
+    } else {
+        DraftNorm n{};
+        n.x16[0] = after;
+        n.w[0] = w + off[D2_POST_NORM];
+        n.out[0] = xn;
+        n.H = H;
+        n.eps = c.rms_eps;
+        launch_rmsnorm16(n, 1, st);
+        g.x = xn;
+    }
     g.N = c.ffn;
     g.K = H;
     g.y16 = act;

@@ -31,8 +31,16 @@ typedef _Float16 half2v_t __attribute__((ext_vector_type(2)));
 // two chunks in flight per wave: 16 loads of 16 bytes per lane, and the x
 // slices of the same chunks read through the cache.  Per-wave sums meet in
 // LDS and are added in a fixed order.
+//
+// NORM: x is the RMSNorm of NORM rows of H inputs (1: of x; 2: of the f32 row
+// nx32, then of x), which every workgroup computes for itself into LDS behind
+// its first weight loads: the normalised row is a few KB through the cache,
+// the weights of a workgroup 64 KB from HBM, and a launch of its own costs the
+// chain 4.7 us (a draft step of three norms: 12 us less in all).  Rows up to 4096 (kGvNormPer pieces of 8 inputs per thread,
+// held beside the weights in flight); wider ones take k_rmsnorm16.
 constexpr int kGvWaves = 4, kGvRows = 8, kGvChunk = 512;
-template <int MODE>
+constexpr int kGvNormPer = 2, kGvNormMax = kGvNormPer * 64 * kGvWaves * 8;
+template <int MODE, int NORM>
 __global__ __launch_bounds__(64 * kGvWaves) void k_gemv16(DraftGemv p) {
     warm_kernargs<sizeof(DraftGemv)>();
     __shared__ float red[kGvWaves][kGvRows];
@@ -46,23 +54,97 @@ __global__ __launch_bounds__(64 * kGvWaves) void k_gemv16(DraftGemv p) {
     }
     const int nrows = MODE == DG_SWIGLU ? 2 * p.N : p.N;
     const rsrc_t wr = make_rsrc(p.w, (uint32_t)((int64_t)nrows * p.K * 2));
-    const rsrc_t xr = make_rsrc(p.x, (uint32_t)p.K * 2);
+    const int nchunk = (p.K + kGvChunk - 1) / kGvChunk;
     float acc[kGvRows];
 #pragma unroll
     for (int r = 0; r < kGvRows; r++) acc[r] = 0.f;
-    const int nchunk = (p.K + kGvChunk - 1) / kGvChunk;
+    uintx4 wv[2][kGvRows], xv[2];
+    auto load_w = [&](int c0, int s) {
+        const int k = (c0 + s * kGvWaves) * kGvChunk + lane * 8;
+#pragma unroll
+        for (int r = 0; r < kGvRows; r++) {
+            const bool ok = k < p.K && row[r] < nrows;
+            wv[s][r] = bld16(wr, ok ? (uint32_t)(((int64_t)row[r] * p.K + k) * 2) : 0x80000000u, 0);
+        }
+    };
+    __shared__ uintx4 xs[NORM ? NORM * kGvNormMax / 8 : 1];  // the normalised x
+    if constexpr (NORM != 0) {
+        __shared__ float ss[NORM][kGvWaves];
+        const int H = p.H;
+        const rsrc_t xr = make_rsrc(p.x, (uint32_t)H * 2);
+        uintx4 xa[NORM][kGvNormPer], wn[NORM][kGvNormPer];
+        uintx4 xf[kGvNormPer][2];
+#pragma unroll
+        for (int i = 0; i < kGvNormPer; i++) {
+            const int e = (i * 64 * kGvWaves + (int)threadIdx.x) * 8;
+            const bool in = e < H;
+            if constexpr (NORM == 2) {
+                const rsrc_t fr = make_rsrc(p.nx32, (uint32_t)H * 4);
+                xf[i][0] = bld16(fr, in ? (uint32_t)e * 4 : 0x80000000u, 0);
+                xf[i][1] = bld16(fr, in ? (uint32_t)e * 4 + 16 : 0x80000000u, 0);
+            }
+            xa[NORM - 1][i] = bld16(xr, in ? (uint32_t)e * 2 : 0x80000000u, 0);
+#pragma unroll
+            for (int n = 0; n < NORM; n++)
+                wn[n][i] = bld16(make_rsrc(p.nw[n], (uint32_t)H * 2), in ? (uint32_t)e * 2 : 0x80000000u, 0);
+        }
+        // these first: a wait for them then leaves the weights in flight
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(wave, 0);
+        load_w(wave, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        auto f16_at = [](const uintx4 &v, int q) {
+            const uint32_t d = v[q >> 1];
+            return h2f((uint16_t)(q & 1 ? d >> 16 : d));
+        };
+        if constexpr (NORM == 2)
+#pragma unroll
+            for (int i = 0; i < kGvNormPer; i++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const uint32_t a = xf[i][q >> 1][2 * (q & 1)], b = xf[i][q >> 1][2 * (q & 1) + 1];
+                    xa[0][i][q] = (uint32_t)f2h(__uint_as_float(a)) | (uint32_t)f2h(__uint_as_float(b)) << 16;
+                }
+#pragma unroll
+        for (int n = 0; n < NORM; n++) {
+            float s = 0.f;
+#pragma unroll
+            for (int i = 0; i < kGvNormPer; i++)
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    const float v = f16_at(xa[n][i], q);
+                    s += v * v;
+                }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+            if (lane == 0) ss[n][wave] = s;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < NORM; n++) {
+            const float ms = ((ss[n][0] + ss[n][1]) + (ss[n][2] + ss[n][3])) / (float)H;
+            const float inv = 1.0f / sqrtf(ms + p.eps);
+#pragma unroll
+            for (int i = 0; i < kGvNormPer; i++) {
+                const int e = (i * 64 * kGvWaves + (int)threadIdx.x) * 8;
+                uintx4 y;
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    y[q] = (uint32_t)f2h(f16_at(xa[n][i], 2 * q) * inv * f16_at(wn[n][i], 2 * q)) |
+                           (uint32_t)f2h(f16_at(xa[n][i], 2 * q + 1) * inv * f16_at(wn[n][i], 2 * q + 1)) << 16;
+                if (e < H) xs[(n * H + e) / 8] = y;
+            }
+        }
+        __syncthreads();
+    }
+    const rsrc_t xr = make_rsrc(p.x, (uint32_t)p.K * 2);
     for (int c0 = wave; c0 < nchunk; c0 += 2 * kGvWaves) {
-        uintx4 wv[2][kGvRows], xv[2];
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             const int k = (c0 + s * kGvWaves) * kGvChunk + lane * 8;
-            const bool kin = k < p.K;
-            xv[s] = bld16(xr, kin ? (uint32_t)k * 2 : 0x80000000u, 0);
-#pragma unroll
-            for (int r = 0; r < kGvRows; r++) {
-                const bool ok = kin && row[r] < nrows;
-                wv[s][r] = bld16(wr, ok ? (uint32_t)(((int64_t)row[r] * p.K + k) * 2) : 0x80000000u, 0);
-            }
+            if constexpr (NORM != 0) xv[s] = k < p.K ? xs[k / 8] : uintx4{0, 0, 0, 0};
+            else xv[s] = bld16(xr, k < p.K ? (uint32_t)k * 2 : 0x80000000u, 0);
+            if (NORM == 0 || c0 != wave) load_w(c0, s);
         }
         // out-of-range loads read zeros, which add nothing
 #pragma unroll
@@ -113,18 +195,24 @@ __global__ __launch_bounds__(64 * kGvWaves) void k_gemv16(DraftGemv p) {
     }
 }
 
+bool gemv16_norm_fits(int H) { return H >= 8 && H % 8 == 0 && H <= kGvNormMax; }
+
 void launch_gemv16(int mode, const DraftGemv &p, hipStream_t st) {
     if (p.K % 8 || p.K < 8 || p.K > kDraftMaxK) throw BackendError("draft gemv: K must be a multiple of 8");
     const int rows = mode == DG_SWIGLU ? 2 * p.N : p.N;
     // weight offsets stay below 2^31 bytes, so the out-of-range sentinel 2^31
     // lies past the buffer resource's size
     if ((int64_t)rows * p.K * 2 >= ((int64_t)1 << 31)) throw BackendError("draft gemv: weight matrix over 2 GiB");
+    if (p.norm && (!gemv16_norm_fits(p.H) || p.K != p.norm * p.H)) throw BackendError("draft gemv: norm width");
     const dim3 grid((rows + kGvRows - 1) / kGvRows), block(64 * kGvWaves);
-    switch (mode) {
-    case DG_STORE: hipLaunchKernelGGL(k_gemv16<DG_STORE>, grid, block, 0, st, p); break;
-    case DG_ADD: hipLaunchKernelGGL(k_gemv16<DG_ADD>, grid, block, 0, st, p); break;
-    case DG_SWIGLU: hipLaunchKernelGGL(k_gemv16<DG_SWIGLU>, grid, block, 0, st, p); break;
-    case DG_LOGITS: hipLaunchKernelGGL(k_gemv16<DG_LOGITS>, grid, block, 0, st, p); break;
+    switch (mode * 4 + p.norm) {
+    case DG_STORE * 4: hipLaunchKernelGGL((k_gemv16<DG_STORE, 0>), grid, block, 0, st, p); break;
+    case DG_STORE * 4 + 2: hipLaunchKernelGGL((k_gemv16<DG_STORE, 2>), grid, block, 0, st, p); break;
+    case DG_ADD * 4: hipLaunchKernelGGL((k_gemv16<DG_ADD, 0>), grid, block, 0, st, p); break;
+    case DG_SWIGLU * 4: hipLaunchKernelGGL((k_gemv16<DG_SWIGLU, 0>), grid, block, 0, st, p); break;
+    case DG_SWIGLU * 4 + 1: hipLaunchKernelGGL((k_gemv16<DG_SWIGLU, 1>), grid, block, 0, st, p); break;
+    case DG_LOGITS * 4: hipLaunchKernelGGL((k_gemv16<DG_LOGITS, 0>), grid, block, 0, st, p); break;
+    case DG_LOGITS * 4 + 1: hipLaunchKernelGGL((k_gemv16<DG_LOGITS, 1>), grid, block, 0, st, p); break;
     default: throw BackendError("draft gemv: mode");
     }
 }

@@ -30,7 +30,15 @@ struct DraftGemv {
     uint16_t *y16;      // STORE / ADD / SWIGLU output (f16)
     const uint16_t *res16;  // ADD: y = f16(f16(W x) + res)
     float *y32;         // LOGITS: the f16 results as f32
+    // norm = 1: the product takes RMSNorm(x) (H inputs, weights nw[0]); 2: the
+    // norms of nx32 (f32, rounded to f16 first; nw[0]) and of x (nw[1]) one
+    // after the other, K = 2 H.  0: x as it is.
+    int norm, H;
+    float eps;
+    const float *nx32;
+    const uint16_t *nw[2];
 };
+bool gemv16_norm_fits(int H);  // else launch_rmsnorm16 first
 void launch_gemv16(int mode, const DraftGemv &p, hipStream_t st);
 
 struct DraftNorm {

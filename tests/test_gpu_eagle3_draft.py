@@ -141,6 +141,22 @@ def test_attention_at_every_step(hip, heads, kv_heads):
     d.close()
 
 
+@pytest.mark.parametrize("hidden,heads,kv_heads", [(256, 1, 1), (2064, 43, 1), (4096, 32, 4), (4608, 36, 4)])
+def test_norms_of_each_width(hip, hidden, heads, kv_heads):
+    """The norms run inside the products up to 4096 inputs (2048 per load, two
+    lanes with a second piece at 2064) and as launches of their own above."""
+    d, c = _draft(hip, hidden=hidden, n_heads=heads, n_kv_heads=kv_heads, ffn=264, draft_vocab=1000)
+    o, _ = _oracle_of(hip, d, c)
+    rng = np.random.default_rng(hidden)
+    for n, s in ((3 * hidden, 0), (hidden, 1)):
+        x, emb = rng.standard_normal(n).astype(np.float32), rng.standard_normal(hidden).astype(np.float32)
+        out_d, lg_d = d.forward_hidden(x, emb, s)
+        out_o = o.forward_hidden(x, emb, s)
+        assert rel_err(out_d, out_o) < TOL, (hidden, s, rel_err(out_d, out_o))
+        assert rel_err(lg_d, o.norm_lm_head(out_o)) < TOL, (hidden, s)
+    d.close()
+
+
 def _target(hip, prefix_len=40, seed=3):
     ocfg = oracle_cfg()
     om = O.OracleModel(ocfg)
