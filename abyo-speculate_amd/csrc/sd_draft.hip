@@ -36,7 +36,7 @@ typedef _Float16 half2v_t __attribute__((ext_vector_type(2)));
 // nx32, then of x), which every workgroup computes for itself into LDS behind
 // its first weight loads: the normalised row is a few KB through the cache,
 // the weights of a workgroup 64 KB from HBM, and a launch of its own costs the
-// chain 4.7 us (a draft step of three norms: 12 us less in all).  Rows up to 4096 (kGvNormPer pieces of 8 inputs per thread,
+// chain 4.7 us (a draft step has three: 10-12 us less in all).  Rows up to 4096 (kGvNormPer pieces of 8 inputs per thread,
 // held beside the weights in flight); wider ones take k_rmsnorm16.
 constexpr int kGvWaves = 4, kGvRows = 8, kGvChunk = 512;
 constexpr int kGvNormPer = 2, kGvNormMax = kGvNormPer * 64 * kGvWaves * 8;
@@ -310,8 +310,7 @@ void launch_from_f16(const uint16_t *x, int64_t n, float *y, hipStream_t st) {
 // loads and cross-lane sums bounds it, so the kernel is compiled for NS steps
 // and NP pairs and the launch takes the least that hold the call's (steps past
 // T add nothing): 10.0 us a launch
-// as one kernel for 16 steps and two pairs, a draft step (with the top-k below)
-// 12 us less.  The values are requested with the keys, not after the scores.
+// as one kernel for 16 steps and two pairs, 4.7 for 4 steps and 6.1 for 8.  The values are requested with the keys, not after the scores.
 constexpr int kAttnPairs = 2;  // head_dim up to 256
 template <int NS, int NP>
 __global__ __launch_bounds__(64) void k_draft_attn(DraftAttn p) {
@@ -450,8 +449,8 @@ void launch_draft_attn(const DraftAttn &p, hipStream_t st) {
 // A (value, index) pair is one 64-bit key whose unsigned order is the selection
 // order, so a round is a maximum over keys: across lanes in four DPP and two
 // permlane-swap steps, where pairs compared field by field through LDS shuffles
-// and the slices' sums added one after the other took 14.5 us at
-// 32 slices.  Outputs the draft ids, l_i - lse, the
+// and the slices' sums added one after the other took 20.6 us
+// on average over calls of 32 and 126 slices (8.3 so).  Outputs the draft ids, l_i - lse, the
 // target ids through d2t, and the top-1 target id as the next step's token.
 constexpr int kTkT = 256, kTkPer = 4, kTkSlice = kTkT * kTkPer, kTkMaxSlices = 256, kTkLaneSlices = kTkMaxSlices / 64;
 static_assert(kTkSlice * kTkMaxSlices >= 262144, "draft top-k slices");
