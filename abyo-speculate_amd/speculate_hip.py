@@ -343,7 +343,8 @@ def _hip_runtime():
         rt.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
         rt.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
         rt.hipHostFree.argtypes = [ctypes.c_void_p]
-        for fn in (rt.hipSetDevice, rt.hipMalloc, rt.hipFree, rt.hipMemcpy, rt.hipHostMalloc, rt.hipHostFree):
+        for fn in (rt.hipSetDevice, rt.hipMalloc, rt.hipFree, rt.hipMemcpy, rt.hipHostMalloc, rt.hipHostFree,
+                   rt.hipGetLastError):
             fn.restype = ctypes.c_int
         _hiprt = rt
     return _hiprt
@@ -380,7 +381,11 @@ class _PinnedPool:
                     rt.hipHostFree(ctypes.c_void_p(self._free[n].pop()))
                     self._pinned -= n
             p = ctypes.c_void_p()
-            if self._pinned + size > self.LIMIT or rt.hipHostMalloc(ctypes.byref(p), size, 1) != 0:  # 1: portable
+            if self._pinned + size > self.LIMIT:
+                return 0
+            if rt.hipHostMalloc(ctypes.byref(p), size, 1) != 0:  # 1: portable
+                # the thread's last error is sticky: left, the next launch that asks for it would report this one
+                rt.hipGetLastError()
                 return 0
             self._pinned += size
             return int(p.value)
