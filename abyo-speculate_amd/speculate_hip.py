@@ -13,6 +13,8 @@ from __future__ import annotations
 
 import collections
 import ctypes
+import errno
+import mmap
 import os
 import threading
 import weakref
@@ -357,7 +359,12 @@ class _PinnedPool:
     30).  A block goes back to the pool when the last array or view on it is
     gone.  At most LIMIT bytes are pinned, blocks in use included; beyond that
     (a caller that keeps many outputs) and for small ones arrays are ordinary.
-    Safe to use from several threads."""
+    Safe to use from several threads.
+
+    The driver does not hand its pages to a forked child, where reading a
+    result would be a segmentation fault: around os.fork the contents of the
+    blocks in use are carried over into ordinary pages at the same addresses
+    (fork_hooks)."""
 
     LIMIT = 256 << 20
     GRAIN = 64 << 10
@@ -365,16 +372,17 @@ class _PinnedPool:
     def __init__(self):
         self._lock = threading.Lock()
         self._free: dict = {}  # block size -> addresses
+        self._used: dict = {}  # address -> block size
         self._pinned = 0
         self._back: collections.deque = collections.deque()  # returned blocks (appended without the lock)
 
     def _take(self, size: int) -> int:
         with self._lock:
-            while self._back:
-                p, n = self._back.popleft()
-                self._free.setdefault(n, []).append(p)
+            self._collect()
             if self._free.get(size):
-                return self._free[size].pop()
+                p = self._free[size].pop()
+                self._used[p] = size
+                return p
             rt = _hip_runtime()
             for n in list(self._free):  # other sizes make room
                 while self._free[n] and self._pinned + size > self.LIMIT:
@@ -388,7 +396,14 @@ class _PinnedPool:
                 rt.hipGetLastError()
                 return 0
             self._pinned += size
+            self._used[int(p.value)] = size
             return int(p.value)
+
+    def _collect(self):
+        while self._back:
+            p, n = self._back.popleft()
+            self._used.pop(p, None)
+            self._free.setdefault(n, []).append(p)
 
     def empty(self, shape, dtype=np.float32) -> np.ndarray:
         count = int(np.prod(shape, dtype=np.int64))
@@ -404,7 +419,50 @@ class _PinnedPool:
         return np.frombuffer(block, dtype, count).reshape(shape)
 
 
+    def fork_hooks(self) -> dict:
+        """The arguments of os.register_at_fork for this pool."""
+        saved = []
+
+        def before():
+            self._lock.acquire()
+            self._collect()
+            saved.extend((p, ctypes.string_at(p, n)) for p, n in self._used.items())
+
+        def parent():
+            saved.clear()
+            self._lock.release()
+
+        def child():
+            try:
+                for p, data in saved:
+                    if _map_pages(p, len(data)):
+                        ctypes.memmove(p, data, len(data))
+            finally:
+                # no HIP in the child: its own arrays are ordinary
+                saved.clear()
+                self._free.clear()
+                self._used.clear()
+                self.LIMIT = 0
+                self._lock.release()
+
+        return dict(before=before, after_in_parent=parent, after_in_child=child)
+
+
+def _map_pages(at: int, size: int) -> bool:
+    """Ordinary zero pages at an address range; False where it is mapped already."""
+    libc = ctypes.CDLL(None, use_errno=True)
+    libc.mmap.restype = ctypes.c_void_p
+    libc.mmap.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
+    fixed_noreplace = 0x100000
+    got = libc.mmap(at, size, mmap.PROT_READ | mmap.PROT_WRITE,
+                    mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS | fixed_noreplace, -1, 0)
+    if got != at and ctypes.get_errno() != errno.EEXIST:
+        raise OSError(ctypes.get_errno(), "result arrays could not be carried over to the forked child")
+    return got == at
+
+
 _pinned = _PinnedPool()
+os.register_at_fork(**_pinned.fork_hooks())
 
 
 class DeviceArray:

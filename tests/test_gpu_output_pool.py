@@ -2,6 +2,7 @@
 were, views keep their block, released blocks are used again, and past the
 bound arrays are ordinary."""
 import gc
+import os
 import threading
 
 import numpy as np
@@ -52,3 +53,27 @@ def test_pool_reuse_bound_and_threads(hip):
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert len(seen) == 800 and all(seen)
+
+
+def test_forked_child_reads_results(hip):
+    """A kept result in a forked child, handed to write(2): EFAULT where its pages did not come along."""
+    ocfg = oracle_cfg(n_layers=1, vocab=32000)
+    dec = hip.HipQuantDecoder(hip_cfg(hip, ocfg))
+    dec.synthesize(MIX_IDS[ocfg.mix], ocfg.seed, ocfg.weight_std)
+    dec.observe([1, 2, 3])
+    for _ in range(4):  # results in blocks that were used before, too
+        rows = dec.batched_logits([4, 5])
+        dec.rollback_to(3)
+    r, w = os.pipe()
+    pid = os.fork()
+    if pid == 0:
+        try:
+            os.write(w, rows.reshape(-1)[-1000:])
+        finally:
+            os._exit(0)
+    os.close(w)
+    with os.fdopen(r, "rb") as f:
+        got = np.frombuffer(f.read(), np.float32)
+    os.waitpid(pid, 0)
+    assert np.array_equal(got, rows.reshape(-1)[-1000:])
+    dec.close()
