@@ -355,49 +355,49 @@ def _hip_runtime():
 class _PinnedPool:
     """Output arrays in pinned host memory: the library's copies into them run
     at the link's speed, where a fresh pageable array costs page faults and a
-    staging copy (5.5 MB of logits: 104 us against 305 us; 0.5 MB: 18 against
-    30).  A block goes back to the pool when the last array or view on it is
-    gone.  At most LIMIT bytes are pinned, blocks in use included; beyond that
-    (a caller that keeps many outputs) and for small ones arrays are ordinary.
-    Safe to use from several threads.
+    staging copy (5.5 MB of logits: 106 us against 317; 0.5 MB: 18 against 32).
+    A block goes back to the pool when the last array or view on it is gone.
+
+    A new block costs far more than it saves once: pinning 0.5 / 2.6 / 5.5 MB
+    takes 0.06-0.3 / 0.13 / 0.12 ms, and the first touch of its pages by the
+    CPU 0.2 / 0.9 / 1.9 ms, against 0.03 / 0.15 / 0.3 ms for the whole copy
+    into an ordinary array.  So a result is never made to wait for one: where
+    no block is free it is an ordinary array, and a pool that is `deferred`
+    adds the block (pinned and touched) at its next grow(), which the decoders
+    call where no result is asked for.  There are at most two blocks of a size
+    class per open decoder and LIMIT bytes in all, blocks in use included; a
+    caller that keeps many outputs gets ordinary arrays from then on, as
+    callers of small ones do.  Closing the last decoder gives the free blocks
+    back, the smallest RETAIN bytes apart, which the next decoder finds warm
+    (release).  Safe to use from several threads; no call into HIP is made with
+    the lock held.
 
     The driver does not hand its pages to a forked child, where reading a
     result would be a segmentation fault: around os.fork the contents of the
     blocks in use are carried over into ordinary pages at the same addresses
-    (fork_hooks)."""
+    (fork_hooks).
+    """
 
     LIMIT = 256 << 20
+    RETAIN = 32 << 20
     GRAIN = 64 << 10
 
-    def __init__(self):
+    def __init__(self, deferred: bool = False):
+        self.deferred = deferred
         self._lock = threading.Lock()
         self._free: dict = {}  # block size -> addresses
         self._used: dict = {}  # address -> block size
+        self._count: dict = {}  # block size -> blocks, free or in use
+        self._want: set = set()  # block sizes that were missed
         self._pinned = 0
+        self._users = 0
         self._back: collections.deque = collections.deque()  # returned blocks (appended without the lock)
 
-    def _take(self, size: int) -> int:
-        with self._lock:
-            self._collect()
-            if self._free.get(size):
-                p = self._free[size].pop()
-                self._used[p] = size
-                return p
-            rt = _hip_runtime()
-            for n in list(self._free):  # other sizes make room
-                while self._free[n] and self._pinned + size > self.LIMIT:
-                    rt.hipHostFree(ctypes.c_void_p(self._free[n].pop()))
-                    self._pinned -= n
-            p = ctypes.c_void_p()
-            if self._pinned + size > self.LIMIT:
-                return 0
-            if rt.hipHostMalloc(ctypes.byref(p), size, 1) != 0:  # 1: portable
-                # the thread's last error is sticky: left, the next launch that asks for it would report this one
-                rt.hipGetLastError()
-                return 0
-            self._pinned += size
-            self._used[int(p.value)] = size
-            return int(p.value)
+    def _size(self, nbytes: int) -> int:
+        """The size class: whole grains, four classes to an octave."""
+        grains = -(-nbytes // self.GRAIN)
+        step = max(0, grains.bit_length() - 3)
+        return (-(-grains >> step) << step) * self.GRAIN
 
     def _collect(self):
         while self._back:
@@ -405,19 +405,85 @@ class _PinnedPool:
             self._used.pop(p, None)
             self._free.setdefault(n, []).append(p)
 
+    def _take(self, size: int) -> int:
+        """A free block of this class or of one up to twice as large, 0 if there is none."""
+        with self._lock:
+            self._collect()
+            for n in [size] + sorted(k for k in self._free if size < k <= 2 * size):
+                if self._free.get(n):
+                    p = self._free[n].pop()
+                    self._used[p] = n
+                    return p
+            if self._may_add(size):
+                self._want.add(size)
+        return 0
+
+    def _may_add(self, size: int) -> bool:
+        return self._count.get(size, 0) < 2 * max(1, self._users) and self._pinned + size <= self.LIMIT
+
+    def grow(self):
+        """Adds a block of each size that was missed since the last call."""
+        while self._want:
+            with self._lock:
+                if not self._want:
+                    return
+                size = self._want.pop()
+                if not self._may_add(size):
+                    continue
+                self._pinned += size
+                self._count[size] = self._count.get(size, 0) + 1
+            rt, p = _hip_runtime(), ctypes.c_void_p()
+            ok = rt.hipHostMalloc(ctypes.byref(p), size, 1) == 0  # 1: portable
+            if ok:
+                ctypes.memset(p, 0, size)
+                self._back.append((int(p.value), size))
+            else:
+                # the thread's last error is sticky: left, the next launch that asks for it would report this one
+                rt.hipGetLastError()
+                with self._lock:
+                    self._pinned -= size
+                    self._count[size] -= 1
+
+    def acquire(self):
+        """A decoder is opened."""
+        with self._lock:
+            self._users += 1
+
+    def release(self):
+        """A decoder is closed; with the last one free blocks are given back."""
+        blocks = []
+        with self._lock:
+            self._users -= 1
+            if self._users > 0:
+                return
+            self._collect()
+            self._want.clear()
+            kept = 0
+            for n in sorted(self._free):
+                while self._free[n] and kept + n * len(self._free[n]) > self.RETAIN:
+                    blocks.append(self._free[n].pop())
+                    self._pinned -= n
+                    self._count[n] -= 1
+                kept += n * len(self._free[n])
+        for p in blocks:
+            _hip_runtime().hipHostFree(ctypes.c_void_p(p))
+
     def empty(self, shape, dtype=np.float32) -> np.ndarray:
         count = int(np.prod(shape, dtype=np.int64))
         nbytes = count * np.dtype(dtype).itemsize
         if nbytes < self.GRAIN // 4:
             return np.empty(shape, dtype)
-        size = -(-nbytes // self.GRAIN) * self.GRAIN
+        size = self._size(nbytes)
         p = self._take(size)
+        if not p and not self.deferred:
+            self.grow()
+            p = self._take(size)
         if not p:
             return np.empty(shape, dtype)
-        block = (ctypes.c_ubyte * size).from_address(p)
-        weakref.finalize(block, self._back.append, (p, size)).atexit = False
+        n = self._used[p]
+        block = (ctypes.c_ubyte * n).from_address(p)
+        weakref.finalize(block, self._back.append, (p, n)).atexit = False
         return np.frombuffer(block, dtype, count).reshape(shape)
-
 
     def fork_hooks(self) -> dict:
         """The arguments of os.register_at_fork for this pool."""
@@ -442,6 +508,7 @@ class _PinnedPool:
                 saved.clear()
                 self._free.clear()
                 self._used.clear()
+                self._want.clear()
                 self.LIMIT = 0
                 self._lock.release()
 
@@ -461,7 +528,7 @@ def _map_pages(at: int, size: int) -> bool:
     return got == at
 
 
-_pinned = _PinnedPool()
+_pinned = _PinnedPool(deferred=True)
 os.register_at_fork(**_pinned.fork_hooks())
 
 
@@ -529,11 +596,13 @@ class HipQuantDecoder:
         self._h = h
         self.vocab = cfg.vocab
         self.hidden = cfg.hidden
+        _pinned.acquire()
 
     def close(self):
         if getattr(self, "_h", None):
             _lib.sd_model_destroy(self._h)
             self._h = None
+            _pinned.release()
 
     def __del__(self):
         try:
@@ -595,6 +664,7 @@ class HipQuantDecoder:
     def observe(self, ids: Sequence[int]):
         a = _u32(ids)
         _check(_lib.sd_observe(self._h, _ptr(a), a.size))
+        _pinned.grow()
 
     def next_logits(self) -> np.ndarray:
         out = _pinned.empty(self.vocab)
@@ -611,6 +681,7 @@ class HipQuantDecoder:
         if n < 0:
             raise ArgError("negative length")
         _check(_lib.sd_rollback_to(self._h, n))
+        _pinned.grow()
 
     def set_eos_token_ids(self, ids: Sequence[int]):
         a = _u32(ids)
@@ -640,6 +711,7 @@ class HipQuantDecoder:
         t, p = tree_arrays(tree)
         a = _u32(accepted)
         _check(_lib.sd_commit_tree_path(self._h, _ptr(t), _ptr(p), t.size, _ptr(a), a.size))
+        _pinned.grow()
 
     def last_hidden_state(self) -> np.ndarray:
         out = _pinned.empty(self.hidden)
