@@ -1,11 +1,13 @@
 // K1 above 16 rows (tree verification, prompts): y[m][n] = sum_k x[m][k] * W[n][k]
 // on v_mfma_f32_32x32x16_f16, weights dequantised to fp16 in registers.
 //
-// A workgroup of 8 waves owns 128 rows (4 row groups of 32) and TT token tiles
-// of 32, for one K slice.  Two waves share a row group: wave half kh multiplies
+// A workgroup owns 128 rows (4 row groups of 32) and TT token tiles of 32, for
+// one K slice.  KH = 2: two waves share a row group, wave half kh multiplies
 // K-chunks 4 kh .. 4 kh + 3 of every superblock, so a SIMD holds two waves
 // (one's dequantisation runs behind the other's MFMAs) and no weight is
 // fetched or dequantised twice; the halves' sums meet in LDS at the end.
+// KH = 1: a wave of its own per row group, and a SIMD's two waves come from two
+// workgroups, for launches of more workgroups than CUs (wide_kh).
 // Activations arrive in operand order (xt_index, sd_common.hpp): a superblock
 // of a token tile is 16 KiB of MFMA operands, 1 KiB each in lane order, so the
 // copy to LDS and every LDS read are contiguous and free of bank conflicts.
@@ -217,7 +219,7 @@ template <> struct WFmt<Q8_0> {
 // The main loop
 // --------------------------------------------------------------------------
 constexpr int kRG = 4;                       // row groups (32 rows each) of a workgroup
-constexpr int kWideThreads = 2 * kRG * 64;   // two chunk halves each
+constexpr int wide_threads(int KH) { return KH * kRG * 64; }  // KH waves share a row group
 constexpr int kXTile = 16384;                // bytes of one token tile's superblock (16 operands of 1 KiB)
 
 struct WideWave {
@@ -229,44 +231,48 @@ struct WideWave {
     int r, j, kh;
 };
 
-template <int FMT, int TT>
+template <int FMT, int TT, int KH>
 __device__ __forceinline__ void wide_body(const WideWave &W, floatx16 (&acc)[TT], uint8_t *lds) {
     typedef WFmt<FMT> F;
     constexpr int STAGE = TT * kXTile;
+    constexpr int PIECE = wide_threads(KH) * 16, PT = kXTile / PIECE;  // bytes of a piece, pieces of a token tile
+    constexpr int HW = 2 / KH, NS = 8 * HW;                            // chunk halves and MFMA steps of a wave
     const int tid = threadIdx.x, lane = tid & 63;
     const int n = W.n;
-    uintx4 xs[2 * TT];
-    typename F::D w[2];
+    uintx4 xs[PT * TT];
+    typename F::D w[2][HW];
     // superblocks past the last are read as the last and not multiplied
     auto ldx = [&](int i, int k) {  // piece k of superblock i's activations
         const uint32_t so = (uint32_t)(min(i, n - 1) + W.sb0) * kXTile;
-        xs[k] = bld16(W.x, (uint32_t)tid * 16u, uni(W.xtile[k >> 1] + so + (uint32_t)(k & 1) * 8192u));
+        xs[k] = bld16(W.x, (uint32_t)tid * 16u, uni(W.xtile[k / PT] + so + (uint32_t)(k % PT) * PIECE));
     };
-    auto ldw = [&](typename F::D &d, int i) {
-        F::load(d, W.w, W.wvo, uni((uint32_t)(min(i, n - 1) + W.sb0) * F::TBB), W.r, W.j, W.kh);
+    auto ldw = [&](typename F::D (&d)[HW], int i) {
+#pragma unroll
+        for (int h = 0; h < HW; h++)
+            F::load(d[h], W.w, W.wvo, uni((uint32_t)(min(i, n - 1) + W.sb0) * F::TBB), W.r, W.j, KH == 2 ? W.kh : h);
     };
-    auto put = [&](int i, int k) {
-        *(uintx4 *)(lds + (i & 1) * STAGE + tid * 16 + k * (kWideThreads * 16)) = xs[k];
-    };
+    auto put = [&](int i, int k) { *(uintx4 *)(lds + (i & 1) * STAGE + tid * 16 + k * PIECE) = xs[k]; };
     // Superblock i is multiplied; between its MFMA steps, a piece at a time, the
     // activations of i + 1 go to the other LDS stage (every wave is past its
     // reads of i - 1 there) and those of i + 2 are requested.  All at the
     // step's start, the copies held the MFMAs up: ffn_down at 128 rows 95 us,
     // 78 so.
-    auto step = [&](const typename F::D &d, int i) {
-        const uint8_t *xb = lds + (i & 1) * STAGE + W.kh * 8192 + lane * 16;
+    auto step = [&](const typename F::D (&d)[HW], int i) {
+        const uint8_t *xb = lds + (i & 1) * STAGE + (KH == 2 ? W.kh * 8192 : 0) + lane * 16;
         typename F::S sc;
-        F::scales(d, sc, W.j, W.kh);
+        F::scales(d[0], sc, W.j, KH == 2 ? W.kh : 0);
         half8 b[2][TT], a[2];
 #pragma unroll
         for (int tt = 0; tt < TT; tt++) b[0][tt] = *(const half8 *)(xb + tt * kXTile);
-        a[0] = F::frag(d, sc, 0, 0);
+        a[0] = F::frag(d[0], sc, 0, 0);
 #pragma unroll
-        for (int ks = 0; ks < 8; ks++) {
-            if (ks < 7) {
+        for (int ks = 0; ks < NS; ks++) {
+            if (ks < NS - 1) {
+                const int kn = ks + 1, h = kn >> 3;
 #pragma unroll
-                for (int tt = 0; tt < TT; tt++) b[(ks + 1) & 1][tt] = *(const half8 *)(xb + tt * kXTile + (ks + 1) * 1024);
-                a[(ks + 1) & 1] = F::frag(d, sc, (ks + 1) >> 1, (ks + 1) & 1);
+                for (int tt = 0; tt < TT; tt++) b[kn & 1][tt] = *(const half8 *)(xb + tt * kXTile + kn * 1024);
+                if (kn == 8) F::scales(d[h], sc, W.j, 1);
+                a[kn & 1] = F::frag(d[h], sc, (kn & 7) >> 1, kn & 1);
             }
             if (ks % (4 / TT) == 0) {
                 put(i + 1, ks / (4 / TT));
@@ -283,15 +289,15 @@ __device__ __forceinline__ void wide_body(const WideWave &W, floatx16 (&acc)[TT]
     // loop is the order inside it.
 #define PIN __builtin_amdgcn_sched_barrier(0)
 #pragma unroll
-    for (int k = 0; k < 2 * TT; k++) ldx(0, k);
+    for (int k = 0; k < PT * TT; k++) ldx(0, k);
     PIN;
     ldw(w[0], 0);
     PIN;
 #pragma unroll
-    for (int k = 0; k < 2 * TT; k++) put(0, k);
+    for (int k = 0; k < PT * TT; k++) put(0, k);
     PIN;
 #pragma unroll
-    for (int k = 0; k < 2 * TT; k++) ldx(1, k);
+    for (int k = 0; k < PT * TT; k++) ldx(1, k);
     PIN;
     ldw(w[1], 1);
     PIN;
@@ -323,8 +329,8 @@ __host__ __device__ inline int wide_groups(const GemmParams &p) {
 // bytes of LDS: two stages of activations, or the sums of two token tiles
 constexpr int kYPitch = 36;                         // floats per token of a 32-row tile (conflict free)
 constexpr int kYTile = 32 * kYPitch;
-template <int TT> constexpr int wide_lds() {
-    const int x = 2 * TT * kXTile, y = 2 * kRG * (TT < 2 ? TT : 2) * kYTile * 4;
+template <int TT, int KH> constexpr int wide_lds() {
+    const int x = 2 * TT * kXTile, y = KH * kRG * (TT < 2 ? TT : 2) * kYTile * 4;
     return x > y ? x : y;
 }
 
@@ -343,8 +349,9 @@ struct WideArgs {
 // nrb row blocks x nks K slices x ntb token blocks; workgroups of one (row
 // block, slice) sit on one XCD one after the other, so the weights leave HBM
 // once and the other token blocks find them in that XCD's L2
-template <int TT, int WPE>
-__global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WPE))) void k_qwide(WideArgs) {
+template <int TT, int KH, int WPE>
+__global__ __launch_bounds__(wide_threads(KH)) __attribute__((amdgpu_waves_per_eu(WPE))) void k_qwide(WideArgs) {
+    constexpr int NT = wide_threads(KH);
     warm_kernargs<sizeof(WideArgs)>();
     const GemmParams &p = kernarg<GemmParams, offsetof(WideArgs, g)>();
     const int nrb = kernarg<int, offsetof(WideArgs, nrb)>(), nks = kernarg<int, offsetof(WideArgs, nks)>(),
@@ -355,9 +362,9 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WP
     const int rb = unit / nks, ks = unit % nks;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool swi = p.mode == GM_SWIGLU;
-    const int nsb = p.K >> 8, m0 = tblk * TT * 32, rg = wave >> 1;
+    const int nsb = p.K >> 8, m0 = tblk * TT * 32, rg = wave / KH;
     WideWave W;
-    W.kh = wave & 1;
+    W.kh = wave % KH;
     W.r = lane & 31;
     W.j = lane >> 5;
     W.sb0 = ks * nsb / nks;
@@ -388,7 +395,7 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WP
     for (int tt = 0; tt < 4; tt++)
         W.xtile[tt] = uni((uint32_t)min((m0 >> 5) + min(tt, TT - 1), last_tile) * (uint32_t)nsb * kXTile);
 
-    // input norm (M <= 64, norm_parts <= 64): thread t's share of token t / 8
+    // input norm (M <= 64, norm_parts <= 64)
     const bool has_norm = p.norm_ssq != nullptr;
     floatx16 acc[TT];
 #pragma unroll
@@ -396,10 +403,10 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WP
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[tt][i] = 0.f;
     switch (S.fmt) {
-    case Q4_K: wide_body<Q4_K, TT>(W, acc, wlds); break;
-    case Q5_K: wide_body<Q5_K, TT>(W, acc, wlds); break;
-    case Q6_K: wide_body<Q6_K, TT>(W, acc, wlds); break;
-    default: wide_body<Q8_0, TT>(W, acc, wlds); break;
+    case Q4_K: wide_body<Q4_K, TT, KH>(W, acc, wlds); break;
+    case Q5_K: wide_body<Q5_K, TT, KH>(W, acc, wlds); break;
+    case Q6_K: wide_body<Q6_K, TT, KH>(W, acc, wlds); break;
+    default: wide_body<Q8_0, TT, KH>(W, acc, wlds); break;
     }
 
     // ---- the sums go through LDS, two token tiles at a time, as [wave][token
@@ -407,13 +414,16 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WP
     // outputs leave in runs of 128 bytes per token ----
     __shared__ float s_inv[64];
     if (has_norm) {
-        float nrm = 0.f;
-        const int m = min(tid >> 3, p.M - 1);
-        for (int q = tid & 7; q < p.norm_parts; q += 8) nrm += p.norm_ssq[m * p.norm_parts + q];
-        nrm += __shfl_xor(nrm, 1);
-        nrm += __shfl_xor(nrm, 2);
-        nrm += __shfl_xor(nrm, 4);
-        if ((tid & 7) == 0) s_inv[tid >> 3] = 1.0f / sqrtf(nrm / (float)p.K + p.norm_eps);
+#pragma unroll
+        for (int t = tid; t < 512; t += NT) {
+            float nrm = 0.f;
+            const int m = min(t >> 3, p.M - 1);
+            for (int q = t & 7; q < p.norm_parts; q += 8) nrm += p.norm_ssq[m * p.norm_parts + q];
+            nrm += __shfl_xor(nrm, 1);
+            nrm += __shfl_xor(nrm, 2);
+            nrm += __shfl_xor(nrm, 4);
+            if ((t & 7) == 0) s_inv[t >> 3] = 1.0f / sqrtf(nrm / (float)p.K + p.norm_eps);
+        }
     }
     constexpr int TR = TT < 2 ? 1 : 2;  // token tiles of a round
     float *Y = (float *)wlds;
@@ -430,8 +440,10 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WP
         __syncthreads();
         // rows 4 c .. 4 c + 3 of group g for token tk of the round
         auto sum = [&](int g, int tk, int c) {
-            const float *y = Y + (2 * g * TR + (tk >> 5)) * kYTile + (tk & 31) * kYPitch + 4 * c;
-            return *(const floatx4 *)y + *(const floatx4 *)(y + TR * kYTile);
+            const float *y = Y + (KH * g * TR + (tk >> 5)) * kYTile + (tk & 31) * kYPitch + 4 * c;
+            floatx4 v = *(const floatx4 *)y;
+            if constexpr (KH == 2) v += *(const floatx4 *)(y + TR * kYTile);
+            return v;
         };
         if (swi) {
             // a thread: token tk, rows 4 c .. of both feature groups -> slots 0..7 of chunk c
@@ -439,7 +451,7 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WP
             const int m = m0 + t0 * 32 + tk, f0 = rb * 64;
             const float inv = has_norm ? s_inv[min(m, 63)] : 1.f;
 #pragma unroll
-            for (int c = tid / (32 * TR); c < 8; c += kWideThreads / (32 * TR)) {
+            for (int c = tid / (32 * TR); c < 8; c += NT / (32 * TR)) {
                 uint32_t o[4];
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
@@ -455,53 +467,58 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WP
             }
             continue;
         }
-        // a thread: rows 4 c .. of one token, the groups in turn (TR == 1: half of them)
-        constexpr int GN = TR == 1 ? kRG / 2 : kRG;
-        const int c = lane & 7, tk = (wave * 8 + (lane >> 3)) & (32 * TR - 1), ga = TR == 1 ? (wave >> 2) * GN : 0;
-        const int m = m0 + t0 * 32 + tk;
-        const bool in = m < p.M;
-        const float inv = has_norm && nks == 1 ? s_inv[min(m, 63)] : 1.f;
-        float bv = -INFINITY;
-        int bi = 0x7fffffff;
+        // a thread: rows 4 c .. of one token, the groups in turn; the NT / 8
+        // tokens at a time are half a round, the round, or the round with the
+        // groups halved
+        constexpr int TP = NT / 8, GS = TP > 32 * TR ? 2 : 1, GN = kRG / GS;
 #pragma unroll
-        for (int g = ga; g < ga + GN; g++) {
-            const int gu = rb * kRG + g;
-            if (!in || gu >= ngr) continue;
-            floatx4 y = sum(g, tk, c);
-            const int n0 = gu * 32 + 4 * c;  // among the launch's rows
-            if (nks > 1) {
-                // K slices: partial sums [ks][M][R]; the consumer of the output adds them in slice order
-                *(floatx4 *)(p.part + ((int64_t)ks * p.M + m) * R + n0) = y;
-                continue;
-            }
-            GemmSeg T = p.seg[0];
+        for (int tp = 0; tp < 32 * TR; tp += TP) {
+            const int c = lane & 7, tk = tp + ((tid >> 3) & (32 * TR - 1)), ga = GS == 2 ? (wave >> 2) * GN : 0;
+            const int m = m0 + t0 * 32 + tk;
+            const bool in = m < p.M;
+            const float inv = has_norm && nks == 1 ? s_inv[min(m, 63)] : 1.f;
+            float bv = -INFINITY;
+            int bi = 0x7fffffff;
 #pragma unroll
-            for (int i = 1; i < 4; i++)
-                if (i < p.nseg && 2 * gu >= p.seg[i].tile0) T = p.seg[i];
-            const int n1 = n0 - T.tile0 * 16;  // in the segment
-            if (has_norm) y *= inv;
-            float *o = T.out + (int64_t)m * T.ldo + T.col0 + n1;
-            if (p.mode == GM_RESID) y += *(const floatx4 *)o;
-            else if (T.bias) y += *(const floatx4 *)(T.bias + n1);
-            *(floatx4 *)o = y;
-            if (p.mode == GM_LOGITS) {
+            for (int g = ga; g < ga + GN; g++) {
+                const int gu = rb * kRG + g;
+                if (!in || gu >= ngr) continue;
+                floatx4 y = sum(g, tk, c);
+                const int n0 = gu * 32 + 4 * c;  // among the launch's rows
+                if (nks > 1) {
+                    // K slices: partial sums [ks][M][R]; the consumer of the output adds them in slice order
+                    *(floatx4 *)(p.part + ((int64_t)ks * p.M + m) * R + n0) = y;
+                    continue;
+                }
+                GemmSeg T = p.seg[0];
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int idx = T.col0 + n1 + i;
-                    if (y[i] > -INFINITY && (y[i] > bv || (y[i] == bv && idx < bi))) {
-                        bv = y[i];
-                        bi = idx;
+                for (int i = 1; i < 4; i++)
+                    if (i < p.nseg && 2 * gu >= p.seg[i].tile0) T = p.seg[i];
+                const int n1 = n0 - T.tile0 * 16;  // in the segment
+                if (has_norm) y *= inv;
+                float *o = T.out + (int64_t)m * T.ldo + T.col0 + n1;
+                if (p.mode == GM_RESID) y += *(const floatx4 *)o;
+                else if (T.bias) y += *(const floatx4 *)(T.bias + n1);
+                *(floatx4 *)o = y;
+                if (p.mode == GM_LOGITS) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int idx = T.col0 + n1 + i;
+                        if (y[i] > -INFINITY && (y[i] > bv || (y[i] == bv && idx < bi))) {
+                            bv = y[i];
+                            bi = idx;
+                        }
                     }
                 }
             }
-        }
-        if (p.mode == GM_LOGITS) {
+            if (p.mode == GM_LOGITS) {
 #pragma unroll
-            for (int o = 1; o < 8; o <<= 1) amax_merge(bv, bi, __shfl_xor(bv, o), __shfl_xor(bi, o));
-            if (c == 0 && in) {
-                const int slot = TR == 1 ? rb * 2 + (wave >> 2) : rb;
-                p.amax_v[(int64_t)m * p.amax_ld + slot] = bv;
-                p.amax_i[(int64_t)m * p.amax_ld + slot] = bi;
+                for (int o = 1; o < 8; o <<= 1) amax_merge(bv, bi, __shfl_xor(bv, o), __shfl_xor(bi, o));
+                if (c == 0 && in) {
+                    const int slot = GS == 2 ? rb * 2 + (wave >> 2) : rb;
+                    p.amax_v[(int64_t)m * p.amax_ld + slot] = bv;
+                    p.amax_i[(int64_t)m * p.amax_ld + slot] = bi;
+                }
             }
         }
     }
@@ -510,9 +527,18 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(WP
 // --------------------------------------------------------------------------
 // Launch policy
 // --------------------------------------------------------------------------
-static int wide_tt(int M) { return M <= 32 ? 1 : M <= 64 ? 2 : 4; }
 static int row_blocks(const GemmParams &p) { return (wide_groups(p) + kRG - 1) / kRG; }
-static int token_blocks(int M) { return (M + 32 * wide_tt(M) - 1) / (32 * wide_tt(M)); }
+static int token_blocks(int M, int tt) { return (M + 32 * tt - 1) / (32 * tt); }
+static bool may_split(const GemmParams &p) { return p.allow_split && (p.mode == GM_STORE || p.mode == GM_RESID); }
+static int wide_tt(const GemmParams &p) { return p.M <= 32 ? 1 : p.M <= 64 ? 2 : 4; }
+static int workgroups(const GemmParams &p) { return row_blocks(p) * token_blocks(p.M, wide_tt(p)); }
+// Waves of a row group.  With two token tiles and more than one workgroup per
+// CU to run, one: its four-wave workgroups sit two to a CU, where the eight-wave
+// ones run in rounds whose prologue and epilogue nothing covers.  At 60 rows
+// of 128256 x 4096 Q4_K (1002 workgroups) 97 us against 105, of gate/up 2 x 18944
+// x 3584 Q8_0 (296) 46 against 49; where every workgroup has a CU of its own two
+// are faster (2 x 14336 x 4096, 224 workgroups: 26.4 against 28.1).
+static int wide_kh(const GemmParams &p) { return wide_tt(p) == 2 && workgroups(p) > 256 ? 1 : 2; }
 // K slices, where the consumer of the output adds them.  Up to 64 rows as many
 // as bring the launch to 192 workgroups (the 60-node tree step at targets of
 // 96 / 128 / 192: 783 / 771 / 737 us).  Above, the count with the least time
@@ -520,8 +546,8 @@ static int token_blocks(int M) { return (M + 32 * wide_tt(M) - 1) / (32 * wide_t
 // 1.9 us a superblock, and the partial sums written and read at 4 TB/s.  280
 // workgroups (3584 rows, 1251 tokens) take two rounds unsplit.
 int qwide_slices(const GemmParams &p) {
-    if (!p.allow_split || (p.mode != GM_STORE && p.mode != GM_RESID)) return 1;
-    const int wgs = row_blocks(p) * token_blocks(p.M), nsb = p.K / 256;
+    if (!may_split(p)) return 1;
+    const int wgs = workgroups(p), nsb = p.K / 256;
     const int64_t R = 16LL * p.ntiles;
     int best = 1;
     double least = 0.0;
@@ -540,39 +566,40 @@ int qwide_slices(const GemmParams &p) {
     }
     return best;
 }
-int qwide_slots(const GemmParams &p) { return row_blocks(p) * (wide_tt(p.M) == 1 ? 2 : 1); }
+int qwide_slots(const GemmParams &p) { return row_blocks(p) * (wide_tt(p) == 1 ? 2 : 1); }
 
-template <int TT, int WPE>
+template <int TT, int KH, int WPE>
 static void wide_launch(const GemmParams &p, hipStream_t st, const LaunchTiming &tm) {
-    const int nrb = row_blocks(p), nks = qwide_slices(p), ntb = token_blocks(p.M);
-    const size_t lds = wide_lds<TT>();
+    const int nrb = row_blocks(p), nks = qwide_slices(p), ntb = token_blocks(p.M, TT);
+    const size_t lds = wide_lds<TT, KH>();
     const WideArgs args{p, nrb, nks, ntb};
-    const dim3 grid((unsigned)((nrb * nks + 7) / 8 * 8 * ntb)), block(kWideThreads);
+    const dim3 grid((unsigned)((nrb * nks + 7) / 8 * 8 * ntb)), block(wide_threads(KH));
     if (lds > 65536) {
         static std::atomic<uint64_t> done{0};  // bit per device
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess) throw BackendError("qwide: hipGetDevice");
         const uint64_t bit = 1ull << (dev & 63);
         if (!(done.load(std::memory_order_acquire) & bit) || dev > 63) {
-            if (hipFuncSetAttribute((const void *)k_qwide<TT, WPE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+            if (hipFuncSetAttribute((const void *)k_qwide<TT, KH, WPE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)lds) != hipSuccess)
                 throw BackendError("qwide: LDS size");
             done.fetch_or(bit, std::memory_order_release);
         }
     }
     if (tm.start && tm.stop)
-        hipExtLaunchKernelGGL((k_qwide<TT, WPE>), grid, block, lds, st, tm.start, tm.stop, 0, args);
-    else hipLaunchKernelGGL((k_qwide<TT, WPE>), grid, block, lds, st, args);
+        hipExtLaunchKernelGGL((k_qwide<TT, KH, WPE>), grid, block, lds, st, tm.start, tm.stop, 0, args);
+    else hipLaunchKernelGGL((k_qwide<TT, KH, WPE>), grid, block, lds, st, args);
 }
 
 void launch_qwide(const GemmParams &p, hipStream_t st, const LaunchTiming &tm) {
     if (qwide_slices(p) > 1 && !p.part) throw BackendError("qgemm: split-K workspace missing");
     for (int i = 0; i < p.nseg; i++)
         if (p.seg[i].rows % 32 || p.seg[i].tile0 % 2) throw BackendError("qgemm: 32-row tiles above 16 tokens");
-    const int tt = wide_tt(p.M);
-    if (tt == 1) wide_launch<1, 4>(p, st, tm);
-    else if (tt == 2) wide_launch<2, 2>(p, st, tm);
-    else wide_launch<4, 2>(p, st, tm);
+    const int tt = wide_tt(p);
+    if (tt == 1) wide_launch<1, 2, 4>(p, st, tm);
+    else if (tt == 4) wide_launch<4, 2, 2>(p, st, tm);
+    else if (wide_kh(p) == 2) wide_launch<2, 2, 2>(p, st, tm);
+    else wide_launch<2, 1, 2>(p, st, tm);
 }
 
 }  // namespace sd

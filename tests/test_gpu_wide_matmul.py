@@ -63,3 +63,37 @@ def test_noalloc_split_unaligned_rows(hip):
             xb.free()
             yb.free()
     dec.close()
+
+
+@pytest.mark.parametrize("mix", ["q4_k", "q5_k", "q6_k", "q8_0"])
+@pytest.mark.parametrize("M", [33, 47, 64])
+def test_more_workgroups_than_cus(hip, mix, M):
+    """33 to 64 rows of more than 256 128-row blocks (257 here, the last one a
+    single 32-row group) take four-wave workgroups: the plain product, and in a
+    tree pass the lm_head with its argmax and gate/up (260 blocks)."""
+    ocfg = oracle_cfg(mix=mix, **dict(SHAPE, ffn=16640, vocab=32800, ctx_len=128))
+    dec = hip.HipQuantDecoder(hip_cfg(hip, ocfg))
+    dec.synthesize(MIX_IDS[mix], ocfg.seed, ocfg.weight_std)
+    fmt, raw = O.synth_tensor(ocfg, -1, O.K_OUTPUT)
+    rows, K = ocfg.shape(O.K_OUTPUT)
+    x = np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)
+    ref = O.round_f16(x).astype(np.float64) @ operand_weights(fmt, raw, rows, K, M).astype(np.float64).T
+    assert rel_err(dec.qmatmul(-1, O.K_OUTPUT, x), ref) < K * 2.0 ** -24 * 8
+    prefix = [5, 6, 7]
+    toks = [7] + [int(v) for v in np.random.default_rng(M).integers(0, ocfg.vocab, M - 1)]
+    tree = (toks, [0] + [max(0, (i - 1) // 3) for i in range(1, M)])
+    dec.observe(prefix)
+    logits, hidden = dec.tree_logits_keep_kv(tree)
+    best = dec.last_argmax(M)
+    assert np.array_equal(best, logits.argmax(1))
+    # the same nodes one root path at a time, on the kernels of up to 16 rows
+    path = []
+    i = M - 1
+    while i:
+        path.append(i)
+        i = tree[1][i]
+    dec.rollback_to(len(prefix))
+    step = dec.batched_logits([toks[j] for j in path[::-1]])
+    # fp16 activations and K-quant weights against exact-integer weights, through one layer
+    assert rel_err(logits[[0] + path[::-1]], step.astype(np.float64)) < 5e-3
+    dec.close()
