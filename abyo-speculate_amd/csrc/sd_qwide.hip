@@ -31,6 +31,7 @@
 // an exact integer sc rounds once) and broadcast by operand selects.
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "sd_buffer.hpp"
@@ -539,24 +540,27 @@ static int workgroups(const GemmParams &p) { return row_blocks(p) * token_blocks
 // x 3584 Q8_0 (296) 46 against 49; where every workgroup has a CU of its own two
 // are faster (2 x 14336 x 4096, 224 workgroups: 26.4 against 28.1).
 static int wide_kh(const GemmParams &p) { return wide_tt(p) == 2 && workgroups(p) > 256 ? 1 : 2; }
-// K slices, where the consumer of the output adds them.  Up to 64 rows as many
-// as bring the launch to 192 workgroups (the 60-node tree step at targets of
-// 96 / 128 / 192: 783 / 771 / 737 us).  Above, the count with the least time
-// by what a launch was measured to cost: rounds of 256 workgroups at 6 us plus
-// 1.9 us a superblock, and the partial sums written and read at 4 TB/s.  280
-// workgroups (3584 rows, 1251 tokens) take two rounds unsplit.
+// K slices, where the consumer of the output adds them.  Up to 64 rows the
+// fewest with which no slice is longer than with the most that run at once, one
+// workgroup to a CU: a 257th starts a second round (4608 x 3584 at 60 rows: 8
+// slices, 288 workgroups 16.5 us, 7 slices 11.3).  Above, the count with the
+// least time by what a launch costs with the chip full: rounds of 256 workgroups
+// at 6 us plus 1.9 us a superblock, and the partial sums written and read at 4
+// TB/s.  280 workgroups (3584 rows, 1251 tokens) take two rounds unsplit.
 int qwide_slices(const GemmParams &p) {
     if (!may_split(p)) return 1;
     const int wgs = workgroups(p), nsb = p.K / 256;
     const int64_t R = 16LL * p.ntiles;
+    auto fits = [&](int ks) { return ks <= 8 && ks <= nsb && (ks == 1 || ks * p.M * R <= p.part_cap); };
+    if (p.M <= 64) {
+        int ks = 1;
+        while (fits(ks + 1) && wgs * (ks + 1) <= 256) ks++;
+        const int longest = (nsb + ks - 1) / ks;
+        return (nsb + longest - 1) / longest;
+    }
     int best = 1;
     double least = 0.0;
-    for (int ks = 1; ks <= 8 && ks <= nsb && (ks == 1 || ks * p.M * R <= p.part_cap); ks *= 2) {
-        if (p.M <= 64) {
-            best = ks;
-            if (wgs * ks >= 192) break;
-            continue;
-        }
+    for (int ks = 1; fits(ks); ks *= 2) {
         const int rounds = (wgs * ks + 255) / 256;
         const double us = rounds * (6.0 + 1.9 * nsb / ks) + (ks > 1 ? ks * p.M * R * 8.0 / 4e6 : 0.0);
         if (ks == 1 || us < least) {

@@ -39,8 +39,8 @@ def test_tile_edges(hip, mix, M):
 
 
 def test_noalloc_split_unaligned_rows(hip):
-    """The allocation-free product with K slices (256 output rows, K = 7168: eight
-    slices) on inputs and outputs that start one float into an allocation."""
+    """The allocation-free product with K slices (256 output rows, K = 7168: seven
+    or eight slices) on inputs and outputs that start one float into an allocation."""
     ocfg = oracle_cfg(mix="q4_k", n_layers=1, hidden=256, n_heads=4, n_kv_heads=1, head_dim=64, ffn=7168, vocab=256,
                       ctx_len=64)
     dec = hip.HipQuantDecoder(hip_cfg(hip, ocfg))
