@@ -531,7 +531,17 @@ __global__ __launch_bounds__(wide_threads(KH)) __attribute__((amdgpu_waves_per_e
 static int row_blocks(const GemmParams &p) { return (wide_groups(p) + kRG - 1) / kRG; }
 static int token_blocks(int M, int tt) { return (M + 32 * tt - 1) / (32 * tt); }
 static bool may_split(const GemmParams &p) { return p.allow_split && (p.mode == GM_STORE || p.mode == GM_RESID); }
-static int wide_tt(const GemmParams &p) { return p.M <= 32 ? 1 : p.M <= 64 ? 2 : 4; }
+// Token tiles of a workgroup: as few as hold the rows, at most four.  Above 64
+// rows a launch of at most 64 workgroups, K slices included, takes two: most
+// CUs are idle, and half the tiles shorten the chain that bounds it (512 wide,
+// 1536 ffn, 96 rows: Q/K/V 8.3 -> 6.5 us, wo 7.6 -> 5.8, gate/up 9.4 -> 7.1,
+// down 8.0 -> 5.9).  Larger launches lose: each weight is dequantised twice
+// (14336 -> 4096 at 96 rows 21.3 -> 22.7).
+static int wide_tt(const GemmParams &p) {
+    if (p.M <= 32) return 1;
+    if (p.M <= 64) return 2;
+    return row_blocks(p) * token_blocks(p.M, 4) * (may_split(p) ? std::min(8, p.K / 256) : 1) <= 64 ? 2 : 4;
+}
 static int workgroups(const GemmParams &p) { return row_blocks(p) * token_blocks(p.M, wide_tt(p)); }
 // Waves of a row group.  With two token tiles and more than one workgroup per
 // CU to run, one: its four-wave workgroups sit two to a CU, where the eight-wave

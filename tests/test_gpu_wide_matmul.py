@@ -97,3 +97,20 @@ def test_more_workgroups_than_cus(hip, mix, M):
     # fp16 activations and K-quant weights against exact-integer weights, through one layer
     assert rel_err(logits[[0] + path[::-1]], step.astype(np.float64)) < 5e-3
     dec.close()
+
+
+def test_small_launches_above_64_rows(hip):
+    """65 to 128 rows of launches that leave most CUs idle take two token tiles
+    a workgroup, with and without K slices."""
+    ocfg = oracle_cfg(mix="q4_k", n_layers=1, hidden=512, n_heads=8, n_kv_heads=8, head_dim=64, ffn=1536, vocab=288,
+                      ctx_len=64)
+    dec = hip.HipQuantDecoder(hip_cfg(hip, ocfg))
+    dec.synthesize(MIX_IDS["q4_k"], ocfg.seed, ocfg.weight_std)
+    for kind in (O.K_ATTN_Q, O.K_FFN_UP, O.K_FFN_DOWN):
+        fmt, raw = O.synth_tensor(ocfg, 0, kind)
+        rows, K = ocfg.shape(kind)
+        for M in (65, 97, 128):
+            x = np.random.default_rng(M + kind).standard_normal((M, K)).astype(np.float32)
+            ref = O.round_f16(x).astype(np.float64) @ operand_weights(fmt, raw, rows, K, M).astype(np.float64).T
+            assert rel_err(dec.qmatmul(0, kind, x), ref) < K * 2.0 ** -24 * 8, (kind, M)
+    dec.close()
