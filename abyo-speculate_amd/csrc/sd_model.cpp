@@ -98,9 +98,10 @@ void Model::alloc_buffers() {
     // many as the context holds), not max_batch: every chunk reads and
     // dequantises all weights and pays the launches, and 128 rows leave the
     // 4096-row matrices with 32 of 256 CUs' worth of tiles.  Above 2048 rows
-    // every matrix fills the chip, so more only costs memory (about 0.2 GB at
-    // the 8B shapes).
-    prompt_rows = std::max(Mx, std::min(kPromptRows, (c.ctx_len + 31) / 32 * 32));
+    // every matrix fills the chip, so more only costs memory (2048 rows take
+    // 0.25 GB more than 128 at the 8B shapes, 0.07 GB of it partial sums).  Handles
+    // of up to 16 rows take prompts in passes of max_batch (advance).
+    prompt_rows = Mx <= 16 ? Mx : std::max(Mx, std::min(kPromptRows, (c.ctx_len + 31) / 32 * 32));
     // rows of the matmuls' inputs: whole 32-token tiles (and 16-token ones + slack)
     const int Rp = prompt_rows, Mp = std::max(128 + 16, (Rp + 31) / 32 * 32);
     cap = ((int64_t)c.ctx_len + 128 + 31) / 32 * 32;  // whole 32-position blocks of the V layout

@@ -137,7 +137,7 @@ class Model {
     int prof_begin();                              // records a start event, returns its index
     void prof_end(int ev, int cls, double bytes);  // records the stop event
 
-    // Most rows of one forward of a prompt, at least max_batch.
+    // Most rows of one forward of a prompt, at least max_batch (max_batch itself up to 16).
     static constexpr int kPromptRows = 2048;
     int prompt_rows = 0;
 

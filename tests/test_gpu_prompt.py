@@ -2,6 +2,8 @@
 forward up to 2048 rows, evenly sized beyond, a remainder of up to 16 rows by
 itself) against the oracle and against the same tokens observed piece by
 piece; the cache rows, the history and what follows the prompt agree too."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -70,3 +72,23 @@ def test_prompt_beyond_one_chunk(hip):
     assert rel_err(a.next_logits(), b.next_logits().astype(np.float64)) < 5e-3
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("max_batch,most", [(16, 96 << 20), (128, 512 << 20)])
+def test_work_buffers_follow_max_batch(hip, max_batch, most):
+    """A handle of up to 16 rows takes prompts in passes of max_batch, and holds
+    no buffers for chunks of 2048 rows (at these widths 0.29 GB beside 17 MB of cache)."""
+    rt = hip._hip_runtime()
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+
+    def left():
+        assert rt.hipDeviceSynchronize() == 0
+        assert rt.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    ocfg = oracle_cfg(ctx_len=4096, n_layers=1, hidden=4096, n_heads=32, n_kv_heads=8, head_dim=128, ffn=14336, vocab=1024)
+    hip.HipQuantDecoder(hip_cfg(hip, ocfg, max_batch=max_batch)).close()  # the library's own allocations
+    before = left()
+    d = hip.HipQuantDecoder(hip_cfg(hip, ocfg, max_batch=max_batch))
+    assert before - left() < most
+    d.close()
