@@ -457,32 +457,11 @@ static GemmSeg seg_of(const DevTensor &t, int tile0, float *out, int ldo, int co
     return s;
 }
 
-void Model::qmatmul(int layer, int kind, const float *x, int M, float *y) {
-    DevTensor &t = slot(*this, layer, kind);
-    if (!t.set() || t.fmt == F32) throw ArgError("qmatmul needs a quantised matrix tensor");
-    if (M < 1 || M > cfg.max_batch) throw ArgError("M out of range");
-    SD_HIP_CHECK(hipSetDevice(cfg.device));
-    float *dx = dalloc<float>((size_t)M * t.K);
-    float *dy = dalloc<float>((size_t)M * t.rows);
-    uint16_t *dxp = dalloc<uint16_t>((size_t)(128 + 16) * t.K);
-    float *part = M > 16 ? dalloc<float>(kNoAllocPartBytes / 4) : nullptr;
-    SD_HIP_CHECK(hipMemcpy(dx, x, (size_t)M * t.K * 4, hipMemcpyHostToDevice));
-    matmul_rows(t, dx, M, dy, dxp, part, st);
-    SD_HIP_CHECK(hipStreamSynchronize(st));
-    SD_HIP_CHECK(hipMemcpy(y, dy, (size_t)M * t.rows * 4, hipMemcpyDeviceToHost));
-    hipFree(dx);
-    hipFree(dy);
-    hipFree(dxp);
-    if (part) hipFree(part);
-}
-
 // Above 16 rows K may be split (a 4096-row matrix alone is 32 workgroups): the
 // slices' sums go to `part` and are added in slice order.  Staging and product
 // of 14336 -> 4096 (Q6_K) at 40 rows: 76.6 us unsplit, 26.5 so; 4096 -> 14336
 // (Q4_K) at 128 rows: 38.3 and 34.3.
-void Model::matmul_rows(const DevTensor &t, const float *x, int M, float *y, uint16_t *staging, float *part,
-                        hipStream_t s) {
-    launch_to_frag16(x, M, t.K, staging, t.K, s);
+static GemmParams rows_params(const DevTensor &t, int M, float *y, const uint16_t *staging, float *part) {
     GemmParams p{};
     p.seg[0] = seg_of(t, 0, y, t.rows, 0, nullptr);
     p.nseg = 1;
@@ -494,6 +473,33 @@ void Model::matmul_rows(const DevTensor &t, const float *x, int M, float *y, uin
     p.allow_split = M > 16;
     p.part = part;
     p.part_cap = kNoAllocPartBytes / 4;
+    return p;
+}
+
+void Model::qmatmul(int layer, int kind, const float *x, int M, float *y) {
+    DevTensor &t = slot(*this, layer, kind);
+    if (!t.set() || t.fmt == F32) throw ArgError("qmatmul needs a quantised matrix tensor");
+    if (M < 1 || M > cfg.max_batch) throw ArgError("M out of range");
+    SD_HIP_CHECK(hipSetDevice(cfg.device));
+    float *dx = dalloc<float>((size_t)M * t.K);
+    float *dy = dalloc<float>((size_t)M * t.rows);
+    uint16_t *dxp = dalloc<uint16_t>((size_t)(128 + 16) * t.K);
+    const int nks = qgemm_slices(rows_params(t, M, dy, dxp, nullptr));
+    float *part = nks > 1 ? dalloc<float>((size_t)nks * M * t.rows) : nullptr;
+    SD_HIP_CHECK(hipMemcpy(dx, x, (size_t)M * t.K * 4, hipMemcpyHostToDevice));
+    matmul_rows(t, dx, M, dy, dxp, part, st);
+    SD_HIP_CHECK(hipStreamSynchronize(st));
+    SD_HIP_CHECK(hipMemcpy(y, dy, (size_t)M * t.rows * 4, hipMemcpyDeviceToHost));
+    hipFree(dx);
+    hipFree(dy);
+    hipFree(dxp);
+    if (part) hipFree(part);
+}
+
+void Model::matmul_rows(const DevTensor &t, const float *x, int M, float *y, uint16_t *staging, float *part,
+                        hipStream_t s) {
+    launch_to_frag16(x, M, t.K, staging, t.K, s);
+    const GemmParams p = rows_params(t, M, y, staging, part);
     launch_qgemm(p, s);
     const int nks = qgemm_slices(p);
     if (nks > 1) launch_add_slices(part, nks, (int64_t)M * t.rows, y, s);

@@ -219,7 +219,7 @@ class Model {
   private:
     void alloc_buffers();
     // y = x . W^T on `s`: staging holds the fp16 rows (whole 32-row tiles above
-    // 16), part kNoAllocPartBytes of K-slice sums
+    // 16), part the K-slice sums (none, or up to kNoAllocPartBytes)
     void matmul_rows(const DevTensor &t, const float *x, int M, float *y, uint16_t *staging, float *part, hipStream_t s);
     void run_gemm(GemmParams &p, int cls, double bytes);
     uint16_t *kc(int layer) const { return kv + (int64_t)layer * 2 * cfg.n_kv_heads * cap * cfg.head_dim; }
