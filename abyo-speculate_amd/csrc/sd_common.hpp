@@ -41,6 +41,7 @@ __host__ __device__ inline int64_t dev_tensor_bytes(int f, int64_t rows, int64_t
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));  // in a caller's rows, which start at any float
 typedef unsigned int uintx4 __attribute__((ext_vector_type(4)));
 typedef unsigned int uintx2 __attribute__((ext_vector_type(2)));
 

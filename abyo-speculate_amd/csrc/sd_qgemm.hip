@@ -433,7 +433,7 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, const GemmSeg (&S)
         } else if (S[rt].bias) {
             r += e.a[rt];
         }
-        *(floatx4 *)o = r;
+        *(floatx4u *)o = r;
         if (p.next_w) {
             // features n .. n+3 sit in fragment slots f, f+2, f+1, f+3 (frag_slot)
             const int n = S[rt].col0 + n0;

@@ -498,9 +498,9 @@ __global__ __launch_bounds__(wide_threads(KH)) __attribute__((amdgpu_waves_per_e
                 const int n1 = n0 - T.tile0 * 16;  // in the segment
                 if (has_norm) y *= inv;
                 float *o = T.out + (int64_t)m * T.ldo + T.col0 + n1;
-                if (p.mode == GM_RESID) y += *(const floatx4 *)o;
+                if (p.mode == GM_RESID) y += *(const floatx4u *)o;
                 else if (T.bias) y += *(const floatx4 *)(T.bias + n1);
-                *(floatx4 *)o = y;
+                *(floatx4u *)o = y;
                 if (p.mode == GM_LOGITS) {
 #pragma unroll
                     for (int i = 0; i < 4; i++) {

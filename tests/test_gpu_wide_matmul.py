@@ -65,6 +65,33 @@ def test_noalloc_split_unaligned_rows(hip):
     dec.close()
 
 
+@pytest.mark.parametrize("M", [5, 17, 40, 128])
+def test_noalloc_unsplit_unaligned_rows(hip, M):
+    """One superblock of K: the product's own stores write the caller's rows,
+    which start 0 to 3 floats into an allocation."""
+    ocfg = oracle_cfg(mix="q4_k", **SHAPE)
+    dec = hip.HipQuantDecoder(hip_cfg(hip, ocfg))
+    dec.synthesize(MIX_IDS["q4_k"], ocfg.seed, ocfg.weight_std)
+    rt = _hip_runtime()
+    for kind in (O.K_ATTN_Q, O.K_FFN_UP):
+        rows, K = ocfg.shape(kind)
+        x = np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)
+        exp = dec.qmatmul(0, kind, x)
+        xb, yb = DevBuf(rt, 4 * M * K), DevBuf(rt, 4 * (M * rows + 8))
+        xb.put(x)
+        for at in range(4):
+            yb.put(np.zeros(M * rows + 8, np.float32))
+            yo = types.SimpleNamespace(p=yb.p.value + 4 * at)
+            assert _noalloc(hip, dec, 0, kind, xb, M, yo) == 0
+            dec.synchronize()
+            got = yb.get(M * rows + 8)
+            assert np.array_equal(got[at:at + M * rows].view(np.uint32), exp.reshape(-1).view(np.uint32)), (kind, at)
+            assert not got[:at].any() and not got[at + M * rows:].any()
+        xb.free()
+        yb.free()
+    dec.close()
+
+
 @pytest.mark.parametrize("mix", ["q4_k", "q5_k", "q6_k", "q8_0"])
 @pytest.mark.parametrize("M", [33, 47, 64])
 def test_more_workgroups_than_cus(hip, mix, M):
