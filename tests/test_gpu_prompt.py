@@ -1,6 +1,6 @@
 """Prompts longer than max_batch: chunks of causal rows through the layers (one
-forward up to 2048 rows, evenly sized beyond, a remainder of up to 16 rows by
-itself) against the oracle and against the same tokens observed piece by
+forward up to 2048 rows, even shares in whole 128-row blocks beyond, a remainder
+of up to 16 rows by itself) against the oracle and against the same tokens observed piece by
 piece; the cache rows, the history and what follows the prompt agree too."""
 import ctypes
 
@@ -57,14 +57,21 @@ def test_prompt_chunks(hip, shape, before, n, max_batch):
     b.close()
 
 
-def test_prompt_beyond_one_chunk(hip):
-    """2113 rows: two chunks of 1057 and 1056 (and 65 = 2113 % 128 rows stay in them)."""
-    ocfg = oracle_cfg(ctx_len=2304, n_layers=1, hidden=256, n_heads=4, n_kv_heads=4, head_dim=64, ffn=256, vocab=1024,
-                      mix="q8_0")
-    ids = [int(v) for v in np.random.default_rng(9).integers(0, ocfg.vocab, 2113)]
+@pytest.mark.parametrize("before,over", [
+    (0, dict(n_heads=4, n_kv_heads=4, mix="q8_0")),
+    (45, dict(n_heads=4, n_kv_heads=2, mix="q4_k")),  # grouped KV heads behind a cached prefix
+], ids=["mha", "gqa-prefix"])
+def test_prompt_beyond_one_chunk(hip, before, over):
+    """2113 rows: the even share rounded up to whole 128-row blocks, 1152, then
+    961 (and 65 = 2113 % 128 rows stay in them)."""
+    ocfg = oracle_cfg(ctx_len=2304, n_layers=1, hidden=256, head_dim=64, ffn=256, vocab=1024, **over)
+    ids = [int(v) for v in np.random.default_rng(9).integers(0, ocfg.vocab, before + 2113)]
     a, b = _dec(hip, ocfg, 128), _dec(hip, ocfg, 128)
-    ha = a.observe_returning_last_hidden(ids)
-    for i in range(0, len(ids), 100):
+    if before:
+        a.observe(ids[:before])
+        b.observe(ids[:before])
+    ha = a.observe_returning_last_hidden(ids[before:])
+    for i in range(before, len(ids), 100):
         hb = b.observe_returning_last_hidden(ids[i:i + 100])
     assert rel_err(ha, hb.astype(np.float64)) < 5e-3
     ka, kb = _kv(a, ocfg, len(ids)), _kv(b, ocfg, len(ids))
