@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2)
 // ---- many queries (tree verify): query tiles across waves, keys shared in LDS ----
 // Grid (kv head, key split, query block).  The kTWaves waves of a workgroup
 // own kTQW query tiles each, the kTWaves * kTQW * 16 queries of one query block
-// of a KV head (all of them up to 256 query rows), and walk the split's keys
+// of a KV head (all of them up to 128 query rows), and walk the split's keys
 // together: each 32-key block of K and V (contiguous in the blocked cache
 // layout) is copied once into LDS by the workgroup's threads and read there by
 // all its waves, so the cache leaves L2 once per query block.  Copies run
@@ -199,10 +199,10 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2)
 // combine kernel merges them.  Eight waves of one tile each: a block of keys
 // costs a workgroup half of what it costs sixteen (each wave reads all of it
 // from LDS), so the same CUs take half the splits in twice the blocks, and half
-// the partial rows are written and merged.  60 rows of 32 heads over 4096 keys,
-// with the merge: 37 us with sixteen waves and 26 splits, 23 with eight and 15
-// (four waves: 25; at 8192 keys 31, 28 and 32; at 1000 keys and 128 rows 22, 19
-// and 21).
+// the partial rows are written and merged.  60 rows of 32 heads, with the merge
+// and the splits of attn_split_wide for both, sixteen against eight waves: over
+// 4096 keys 27.1 and 21.7 us, 8192 31.3 and 28.6, 1000 19.4 and 16.0 (128 rows
+// 22.0 and 19.2).
 constexpr int kTWaves = 8;
 constexpr int kTThreads = 64 * kTWaves;
 constexpr int kTQW = 1;
@@ -433,9 +433,12 @@ void launch_rope_kv(const RopeKvParams &p, hipStream_t st) {
     hipLaunchKernelGGL(k_rope_kv, dim3(p.M, (units + 63) / 64), dim3(64), 0, st, p);
 }
 
-// k_attn_t: splits of whole 32-key blocks, as many as the query blocks leave
-// CUs for (a workgroup fills a CU; one workgroup more than CUs is a second round:
-// 90 rows over 300 keys 15.2 against 19.6 us)
+// k_attn_t: splits of whole 32-key blocks, as many as leave each workgroup a CU
+// of its own.  At head_dim 128 (140 VGPRs) a workgroup fills a CU and one more
+// than CUs is a second round: counted from P + 1 keys instead of P + M, 4155 keys
+// made 33 splits and 264 sixteen-wave workgroups of 60 rows, 36.4 us against
+// 27.1 with 26 splits; 90 rows over 300 keys 19.6 against 15.2.  At head_dim 64
+// (87 VGPRs) two would fit; the count is the same.
 AttnSplit attn_split_wide(int P, int M, int n_kv, int n_rep, int max_splits) {
     const int T = P + M, nqt = (M * n_rep + 15) / 16, nqb = (nqt + kTWaves * kTQW - 1) / (kTWaves * kTQW);
     const int want = std::max(1, std::min(max_splits, 256 / (n_kv * nqb)));

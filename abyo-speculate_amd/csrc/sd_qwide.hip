@@ -16,8 +16,11 @@
 // each with the whole chip busy, when it clocks at 1.9 GHz) against about 17
 // other vector instructions per MFMA step (2 ns each), which issue beside
 // another wave's MFMAs but not beside their own wave's: instruction issue up to
-// 64 rows, the MFMAs above (a superblock of 128 rows and 128 tokens takes 1.28 us, its
-// MFMAs 1.09).  A launch adds 6 us.  Gate/up of 2 x 14336 x 4096
+// 64 rows (a superblock of 128 rows and 64 tokens takes 0.9 us with 64
+// workgroups running, 1.0 with 256, its MFMAs 0.55), the MFMAs most of it above
+// (128 tokens: 1.3 us with 128 workgroups, 1.5 with 256 and 1.65 for Q6_K and
+// Q8_0, against 1.09).  A launch adds 5 to 9 us, of which the outputs' stores
+// are most.  Gate/up of 2 x 14336 x 4096
 // Q4_K (weights in the caches) at 27 / 60 / 128 rows: 18.7 / 21.5 / 32.2 us,
 // where one 16-row tile per wave with the activations in row order took
 // 23.8 / 33.1 / 55.7 us; at 512 rows 148 us (812 TFLOP/s).
@@ -554,9 +557,13 @@ static int wide_kh(const GemmParams &p) { return wide_tt(p) == 2 && workgroups(p
 // fewest with which no slice is longer than with the most that run at once, one
 // workgroup to a CU: a 257th starts a second round (4608 x 3584 at 60 rows: 8
 // slices, 288 workgroups 16.5 us, 7 slices 11.3).  Above, the count with the
-// least time by what a launch costs with the chip full: rounds of 256 workgroups
-// at 6 us plus 1.9 us a superblock, and the partial sums written and read at 4
-// TB/s.  280 workgroups (3584 rows, 1251 tokens) take two rounds unsplit.
+// least modelled time: rounds of 256 workgroups at 6 us plus 1.9 us a
+// superblock, and the partial sums written and read at 4 TB/s.  280 workgroups
+// (3584 rows, 1251 tokens) take two rounds unsplit.  The weights are those that
+// chose best, not a launch's own: full rounds measured 9.3 us plus 1.5 (Q4_K)
+// to 1.67 us (Q8_0), but with 9.3 and 1.6 the rule took 1 slice for 4 (600 rows
+// of 18944 -> 3584: 131 against 119 us, that prompt 2016 against 1971) and won
+// nowhere above 64 rows by more than the runs differ.
 int qwide_slices(const GemmParams &p) {
     if (!may_split(p)) return 1;
     const int wgs = workgroups(p), nsb = p.K / 256;
