@@ -595,7 +595,7 @@ static void wide_launch(const GemmParams &p, hipStream_t st, const LaunchTiming 
     const size_t lds = wide_lds<TT, KH>();
     const WideArgs args{p, nrb, nks, ntb};
     const dim3 grid((unsigned)((nrb * nks + 7) / 8 * 8 * ntb)), block(wide_threads(KH));
-    if (lds > 65536) {
+    if (lds + sizeof(float) * 64 > 65536) {  // with s_inv
         static std::atomic<uint64_t> done{0};  // bit per device
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess) throw BackendError("qwide: hipGetDevice");
