@@ -14,6 +14,7 @@ from __future__ import annotations
 import collections
 import ctypes
 import errno
+import math
 import mmap
 import os
 import threading
@@ -409,11 +410,13 @@ class _PinnedPool:
         """A free block of this class or of one up to twice as large, 0 if there is none."""
         with self._lock:
             self._collect()
-            for n in [size] + sorted(k for k in self._free if size < k <= 2 * size):
-                if self._free.get(n):
-                    p = self._free[n].pop()
-                    self._used[p] = n
-                    return p
+            n = size
+            if not self._free.get(n):
+                n = min((k for k, ps in self._free.items() if ps and size < k <= 2 * size), default=0)
+            if n:
+                p = self._free[n].pop()
+                self._used[p] = n
+                return p
             if self._may_add(size):
                 self._want.add(size)
         return 0
@@ -469,7 +472,7 @@ class _PinnedPool:
             _hip_runtime().hipHostFree(ctypes.c_void_p(p))
 
     def empty(self, shape, dtype=np.float32) -> np.ndarray:
-        count = int(np.prod(shape, dtype=np.int64))
+        count = math.prod(shape) if isinstance(shape, tuple) else int(shape)
         nbytes = count * np.dtype(dtype).itemsize
         if nbytes < self.GRAIN // 4:
             return np.empty(shape, dtype)
