@@ -90,7 +90,7 @@ typedef struct sd_config {
     float rope_theta;     /* rope.freq_base */
     float rms_eps;        /* attention.layer_norm_rms_epsilon */
     int32_t ctx_len;      /* KV capacity in positions (context_length) */
-    int32_t max_batch;    /* rows of one verify pass (<= 128); observes beyond it take chunks of up to 2048 rows */
+    int32_t max_batch;    /* rows of one verify pass (<= 128); above 16, observes beyond it take chunks of up to 2048 rows */
     int32_t tied_output;  /* 1: lm_head reuses token_embd (quantized_llama_local.rs:249-252) */
     int32_t device;       /* HIP device ordinal */
 } sd_config;
