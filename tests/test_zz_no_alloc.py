@@ -146,3 +146,39 @@ def test_noalloc_rejects_inputs_beyond_the_scratch(hip):
             yb.free()
     finally:
         dec.close()
+
+
+@pytest.mark.parametrize("kind,rows", [(3, 5), (9, 40), (9, 128), (7, 33)])
+def test_noalloc_under_capture(hip, kind, rows):
+    """Recorded into a graph and replayed on new inputs, eager calls in between."""
+    ocfg = oracle_cfg(mix="q4_k_m", n_layers=2, vocab=2048, ffn=2048)
+    dec = hip.HipQuantDecoder(hip_cfg(hip, ocfg))
+    dec.synthesize(MIX_IDS["q4_k_m"], ocfg.seed, ocfg.weight_std)
+    dec.synchronize()
+    rt = _hip_runtime()
+    P = ctypes.c_void_p
+    rt.hipStreamBeginCapture.argtypes = [P, ctypes.c_int]
+    rt.hipStreamEndCapture.argtypes = [P, ctypes.POINTER(P)]
+    rt.hipGraphInstantiate.argtypes = [ctypes.POINTER(P), P, P, P, ctypes.c_size_t]
+    rt.hipGraphLaunch.argtypes = [P, P]
+    rt.hipGraphExecDestroy.argtypes = rt.hipGraphDestroy.argtypes = [P]
+    N, K = ocfg.shape(kind)
+    xb, yb = DevBuf(rt, rows * K * 4), DevBuf(rt, rows * N * 4)
+    stream, graph, ex = P(), P(), P()
+    assert rt.hipStreamCreate(ctypes.byref(stream)) == 0
+    assert rt.hipStreamBeginCapture(stream, 0) == 0
+    rc = _noalloc(hip, dec, 1, kind, xb, rows, yb, stream)
+    assert rt.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0 and rc == 0
+    assert rt.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, 0) == 0
+    for i in range(4):
+        x = np.random.default_rng(i).standard_normal((rows, K)).astype(np.float32)
+        xb.put(x)
+        assert rt.hipGraphLaunch(ex, stream) == 0 and rt.hipStreamSynchronize(stream) == 0
+        got = yb.get((rows, N))
+        assert np.array_equal(got.view(np.uint32), dec.qmatmul(1, kind, x).view(np.uint32)), i
+    rt.hipGraphExecDestroy(ex)
+    rt.hipGraphDestroy(graph)
+    rt.hipStreamDestroy(stream)
+    xb.free()
+    yb.free()
+    dec.close()
