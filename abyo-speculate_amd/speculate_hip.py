@@ -17,6 +17,7 @@ import errno
 import math
 import mmap
 import os
+import sys
 import threading
 import weakref
 from dataclasses import dataclass
@@ -507,12 +508,13 @@ class _PinnedPool:
                     if _map_pages(p, len(data)):
                         ctypes.memmove(p, data, len(data))
             finally:
-                # no HIP in the child: its own arrays are ordinary
+                # no HIP in the child: its own arrays are ordinary, and no block is freed
                 saved.clear()
                 self._free.clear()
                 self._used.clear()
                 self._want.clear()
                 self.LIMIT = 0
+                self.RETAIN = sys.maxsize
                 self._lock.release()
 
         return dict(before=before, after_in_parent=parent, after_in_child=child)

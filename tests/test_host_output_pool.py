@@ -82,10 +82,16 @@ def test_results_are_readable_in_a_forked_child(runtime):
     a[:], b[:] = 3.5, -1.0
     view, gone = a[5], pool.empty((300, 1000))
     del a, gone
+    pool.RETAIN = 0
 
     def probe():
+        nonlocal b
         ok = (view == 3.5).all() and (b == -1.0).all() and pool.empty((64, 1000)).flags.owndata
         view[:] = 9.0
+        b = None  # a carried-over block that comes back is not the child's to free
+        pool.acquire()
+        pool.release()
+        ok = ok and len(runtime.blocks) == 2
         return b"same" if ok else b"other"
 
     try:
@@ -94,6 +100,7 @@ def test_results_are_readable_in_a_forked_child(runtime):
         del b
         assert not pool.empty(70000).flags.owndata  # the parent's pool goes on
     finally:
+        del pool.RETAIN
         for d in (pool._free, pool._used, pool._count, pool._want):
             d.clear()
         pool._pinned = 0
