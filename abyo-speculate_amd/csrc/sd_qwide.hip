@@ -19,8 +19,8 @@
 // 64 rows (a superblock of 128 rows and 64 tokens takes 0.9 us with 64
 // workgroups running, 1.0 with 256, its MFMAs 0.55), the MFMAs most of it above
 // (128 tokens: 1.3 us with 128 workgroups, 1.5 with 256 and 1.65 for Q6_K and
-// Q8_0, against 1.09).  A launch adds 5 to 9 us, of which the outputs' stores
-// are most.  Gate/up of 2 x 14336 x 4096
+// Q8_0, against 1.09).  A launch adds 4 to 9 us, the more the more it stores (9
+// with 17 MB of outputs).  Gate/up of 2 x 14336 x 4096
 // Q4_K (weights in the caches) at 27 / 60 / 128 rows: 18.7 / 21.5 / 32.2 us,
 // where one 16-row tile per wave with the activations in row order took
 // 23.8 / 33.1 / 55.7 us; at 512 rows 148 us (812 TFLOP/s).
